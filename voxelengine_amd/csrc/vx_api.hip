@@ -1432,10 +1432,23 @@ static vx_status enqueue_trace_march(vx_ctx* ctx, const vx_volume* vol, const Tr
     MarchShape sh;
     if (vx_status st = march_shape(ctx, true, sh)) return st;
     set_bands(A, sh.grid * (uint32_t)(sh.block / 64));
+    // no more waves than queue items: waves without one only cost the queue
+    sh.grid = std::min<uint32_t>(sh.grid, 8 * cdiv(A.band, sh.block / 64));
     hipLaunchKernelGGL(k_zero_u32, dim3(cdiv(kCounterWords, 256)), dim3(256), 0, stream, A.counters, (int)kCounterWords);
     hipError_t e = launch_march(sh.block, sh.steps, true, sh.grid, sh.rest_grid, stream, A, e0, e1);
     if (e == hipSuccess) e = launch_status();
     if (e != hipSuccess) return fail(VX_ERR_DEVICE, "launch of the ray-parallel trace failed: %s", hipGetErrorString(e));
+    return VX_OK;
+}
+
+// A pair of events for a profiled launch, kept by the context.
+static vx_status profile_events(vx_ctx* ctx, hipEvent_t& e0, hipEvent_t& e1) {
+    VX_HIP(hipEventCreate(&e0));
+    if (hipError_t ce = hipEventCreate(&e1)) {
+        (void)hipEventDestroy(e0);
+        return fail(VX_ERR_DEVICE, "hipEventCreate failed: %s", hipGetErrorString(ce));
+    }
+    ctx->prof.emplace_back(e0, e1);
     return VX_OK;
 }
 
@@ -1448,14 +1461,8 @@ static vx_status launch_trace_march(vx_ctx* ctx, const vx_volume* vol, const Tra
     if (vx_status st = ensure_march(ctx->march, slots, T.fetches != nullptr)) return st;
     MarchScratch M = {ctx->march.res, ctx->march.deferred, ctx->march.fres, ctx->march.counters};
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (ctx->profile) {
-        VX_HIP(hipEventCreate(&e0));
-        if (hipError_t ce = hipEventCreate(&e1)) {
-            (void)hipEventDestroy(e0);
-            return fail(VX_ERR_DEVICE, "hipEventCreate failed: %s", hipGetErrorString(ce));
-        }
-        ctx->prof.emplace_back(e0, e1);
-    }
+    if (ctx->profile)
+        if (vx_status st = profile_events(ctx, e0, e1)) return st;
     return enqueue_trace_march(ctx, vol, T, 0, ntiles, M, stream, e0, e1, hits);
 }
 
@@ -1480,6 +1487,34 @@ static vx_status launch_trace_march_noalloc(vx_ctx* ctx, const vx_volume* vol, c
         const uint32_t n = std::min(chunk, ntiles - t0);
         if (vx_status st = enqueue_trace_march(ctx, vol, T, t0, n, M, stream, nullptr, nullptr)) return st;
     }
+    return VX_OK;
+}
+
+// A whole view with k_trace_tile, `waves` waves per tile: one kernel, no scratch.
+static vx_status launch_trace_tile_view(vx_ctx* ctx, const vx_volume* vol, const TraceArgs& T, const TileGeom& g,
+                                        uint32_t waves, hipStream_t stream) {
+    MarchArgs A;
+    std::memset(&A, 0, sizeof(A));
+    A.item0 = make_march_item(vol, T, 0u, g);
+    A.nrays = T.params.n_shadow + T.params.n_ao + T.params.n_spec;
+    A.ntiles = g.ntiles;
+    A.band_tiles = cdiv(g.ntiles, 8);
+    A.last_word = (uint32_t)(vol->ngrid - 1);
+    const vx_trace_params& p = T.params;
+    const int32_t n[3] = {p.n_shadow, p.n_ao, p.n_spec}, m[3] = {p.shadow_march, p.ao_march, p.spec_march};
+    bool dda = false, sparse = false;
+    for (int k = 0; k < 3; ++k) {
+        dda = dda || (n[k] > 0 && m[k] == VX_MARCH_DDA);
+        sparse = sparse || (n[k] > 0 && m[k] != VX_MARCH_DDA);
+    }
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (ctx->profile && !sparse)
+        if (vx_status st = profile_events(ctx, e0, e1)) return st;
+    hipError_t e = e0 ? hipEventRecord(e0, stream) : hipSuccess;
+    if (e == hipSuccess) e = launch_trace_tile(dda, sparse, waves, stream, A);
+    if (e == hipSuccess && e1) e = hipEventRecord(e1, stream);
+    if (e == hipSuccess) e = launch_status();
+    if (e != hipSuccess) return fail(VX_ERR_DEVICE, "launch of k_trace_tile failed: %s", hipGetErrorString(e));
     return VX_OK;
 }
 
@@ -1524,6 +1559,12 @@ static vx_status trace_impl(vx_ctx* ctx, const vx_volume* vol, const vx_view* vi
             VX_LAUNCHED("k_fill_u64");
         }
         return launch_trace_march(ctx, vol, A, S(stream), hits);
+    }
+    // small launches without fetch counts (the tile kernel keeps none)
+    if (ctx->tuning.kernel == 0 && !A.fetches) {
+        const TileGeom g = tile_geom(ctx->tuning, view->width, view->height);
+        const uint32_t waves = trace_tile_waves(g.ntiles, params->n_shadow + params->n_ao + params->n_spec, all_dda);
+        if (waves) return launch_trace_tile_view(ctx, vol, A, g, waves, S(stream));
     }
     if (all_dda && ctx->tuning.kernel != 1)
         return noalloc ? launch_trace_march_noalloc(ctx, vol, A, S(stream)) : launch_trace_march(ctx, vol, A, S(stream));
@@ -2007,14 +2048,8 @@ static vx_status vx_batch_launch_direct_impl(vx_batch* b, void* stream) {
     if (vx_status st = use_device(b->ctx)) return st;
     vx_ctx* ctx = b->ctx;
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (ctx->profile) {
-        VX_HIP(hipEventCreate(&e0));
-        if (hipError_t ce = hipEventCreate(&e1)) {
-            (void)hipEventDestroy(e0);
-            return fail(VX_ERR_DEVICE, "hipEventCreate failed: %s", hipGetErrorString(ce));
-        }
-        ctx->prof.emplace_back(e0, e1);
-    }
+    if (ctx->profile)
+        if (vx_status st = profile_events(ctx, e0, e1)) return st;
     hipError_t e = batch_enqueue(b, S(stream), e0, e1);
     if (e != hipSuccess) return fail(VX_ERR_DEVICE, "batch launch failed: %s", hipGetErrorString(e));
     return VX_OK;

@@ -77,6 +77,7 @@ struct MarchArgs {
     int32_t nrays;
     int32_t refill;            // not-running lanes that trigger a refill
     float maxt[3];             // shadow, AO, spec
+    uint32_t last_word;        // index of the march grid's last word (k_trace_tile)
 };
 
 struct LightArgs {
@@ -284,6 +285,8 @@ __global__ void k_mgrid(uint64_t* grid, OccView V, int32_t gx, int32_t gy, int32
 // steps between refills; launch_march enqueues march, listed rays and resolve
 // (e0 / e1, when given, are recorded around the march kernel).
 const void* march_kernel(int block, int steps, bool single);
+uint32_t trace_tile_waves(uint32_t ntiles, int32_t nrays, bool all_dda);
+hipError_t launch_trace_tile(bool dda, bool sparse, uint32_t waves, hipStream_t s, const MarchArgs& A);
 hipError_t launch_march(int block, int steps, bool single, uint32_t grid, uint32_t rest_grid, hipStream_t s,
                         const MarchArgs& A, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 

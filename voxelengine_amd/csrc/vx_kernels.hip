@@ -12,6 +12,8 @@
 //                                             LightAmbient.frag:178-214, PBR.frag:3-68
 #include "vx_internal.hpp"
 
+#include <algorithm>
+
 namespace vx {
 
 // ===========================================================================
@@ -645,7 +647,7 @@ VXD void trace_pixel_exact(const OccView& V, const TraceArgs& A, size_t i) {
     uint8_t lit = 1;
     if (P.n_shadow > 0) {
         int32_t h;
-        float t = march_dist(V, P.shadow_march, org, wd, P.shadow_maxt, nf, h);
+        float t = march_dist<kSparsePrefetch>(V, P.shadow_march, org, wd, P.shadow_maxt, nf, h);
         if (P.shadow_march == VX_MARCH_DDA) lit = h ? 0 : 1;
         else lit = (t != P.shadow_maxt) ? 0 : 1;
     }
@@ -663,7 +665,8 @@ VXD void trace_pixel_exact(const OccView& V, const TraceArgs& A, size_t i) {
             f3 dir = mk3((T.x * rv.x + B.x * rv.y) + n.x * rv.z, (T.y * rv.x + B.y * rv.y) + n.y * rv.z,
                          (T.z * rv.x + B.z * rv.y) + n.z * rv.z);
             int32_t h;
-            float t = march_dist(V, P.ao_march, org, dir, P.ao_maxt, nf, h);
+            float t = P.ao_maxt > 16.0f ? march_dist<kSparsePrefetch>(V, P.ao_march, org, dir, P.ao_maxt, nf, h)
+                                        : march_dist(V, P.ao_march, org, dir, P.ao_maxt, nf, h);
             float q = gmin(t, P.ao_maxt) / P.ao_maxt;
             aosum = aosum + q * q;
         }
@@ -695,7 +698,7 @@ VXD void trace_pixel_exact(const OccView& V, const TraceArgs& A, size_t i) {
         f3 wdir = mk3(I.x - (2.0f * dhi) * h.x, I.y - (2.0f * dhi) * h.y, I.z - (2.0f * dhi) * h.z);
         f3 so = mk3((pp.x + n.x * u3) + n.x, (pp.y + n.y * u3) + n.y, (pp.z + n.z * u3) + n.z);
         int32_t hh;
-        float t = march_dist(V, P.spec_march, so, wdir, P.spec_maxt, nf, hh);
+        float t = march_dist<kSparsePrefetch>(V, P.spec_march, so, wdir, P.spec_maxt, nf, hh);
         spv = gmin(t, P.spec_maxt) / P.spec_maxt;
     }
     A.spec[i] = spv;
@@ -1086,6 +1089,14 @@ k_march(MarchArgs A) {
     static_assert(256 % STEPS == 0, "the step limit is tested at block ends");
     constexpr int WAVES = BLOCK / 64;
     __shared__ uint32_t ring_s[WAVES][kRingFields][kRing];
+    // bands found empty: by any wave of the block, or (512 threads, whose rings
+    // leave no LDS at four blocks per CU) by the wave itself
+    __shared__ uint32_t empty_s;
+    uint32_t empty = 0;
+    if (BLOCK == 256) {
+        if (threadIdx.x == 0) empty_s = 0;
+        __syncthreads();
+    }
     const uint32_t lane = threadIdx.x & 63u;
     uint32_t(*ring)[kRing] = ring_s[threadIdx.x >> 6];
     const int32_t nrays = A.nrays;
@@ -1093,7 +1104,7 @@ k_march(MarchArgs A) {
 
     // generation cursor (wave-uniform): queue item = (tile, chunk of its
     // rays); gr runs over the chunk's generation indices [gr, gend)
-    uint32_t q = blockIdx.x & 7u, misses = 0;
+    uint32_t q = blockIdx.x & 7u;
     bool gen_done = nrays <= 0;   // no rays per pixel: k_resolve writes the defaults
     uint32_t gitem = 0, gtile = 0;
     int32_t gr = SINGLE ? 0 : nrays, gend = 0;
@@ -1183,27 +1194,39 @@ k_march(MarchArgs A) {
                     if (!pending) {
                         // next queue item: own band first, then the others. A
                         // band is its tile range once per chunk; the last band's
-                        // items past the last tile are skipped.
+                        // items past the last tile are skipped. A wave that finds
+                        // a band empty marks it for its block: atomics on one
+                        // counter serialize at about 12 ns, and a launch whose
+                        // every wave tried every band ended 90 us late.
                         uint32_t tile = 0, chunk = 0;
                         bool got = false;
-                        while (misses < 8u) {
+                        while (true) {
+                            if (BLOCK == 256)
+                                empty = __builtin_amdgcn_readfirstlane(
+                                    __hip_atomic_load(&empty_s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+                            const uint32_t left = ~empty & 0xffu;
+                            if (left == 0) break;
+                            // the first one from q on
+                            q = (q + (uint32_t)__builtin_ctz(left >> q | left << (8u - q))) & 7u;
                             uint32_t t = 0;
                             if (lane == 0) t = atomicAdd(&A.counters[q * kCounterStride], 1u);
                             t = __builtin_amdgcn_readfirstlane(t);
-                            if (SINGLE) {
-                                if (t < A.band) {
+                            if (t < A.band) {
+                                if (SINGLE) {
                                     chunk = t / A.band_tiles;
                                     tile = q * A.band_tiles + (t - chunk * A.band_tiles);
-                                    if (tile < A.ntiles) { got = true; break; }
-                                    continue;
+                                } else {
+                                    // a batch takes one item per tile
+                                    tile = q * A.band + t;
                                 }
-                            } else {
-                                // a batch takes one item per tile
-                                tile = q * A.band + t;
-                                if (t < A.band && tile < A.ntiles) { got = true; break; }
+                                if (tile < A.ntiles) { got = true; break; }
+                                if (SINGLE) continue;
                             }
-                            q = (q + 1u) & 7u;
-                            misses++;
+                            if (BLOCK == 256) {
+                                if (lane == 0) atomicOr(&empty_s, 1u << q);
+                            } else {
+                                empty |= 1u << q;
+                            }
                         }
                         if (!got) { gen_done = true; break; }
                         gtile = tile;
@@ -1463,6 +1486,210 @@ __global__ void __launch_bounds__(256) k_resolve(MarchArgs A) {
     T.ao[i] = P.n_ao > 0 ? aosum / (float)P.n_ao : 1.0f;
     T.spec[i] = P.n_spec > 0 ? spv : 1.0f;
     if (T.fetches) T.fetches[i] = nf;
+}
+
+// ===========================================================================
+// The trace of a small launch: one block per 64-pixel tile, its waves taking
+// the tile's rays one ray index at a time (long classes first), one ray per
+// lane, results folded in LDS by the wave that ends last (the others leave and
+// free their slots). A launch of few rays lasts as long as its longest ray, so
+// what counts is the latency of a step and of the launch: no queue, no ring,
+// no scratch, one kernel, and the marches read ahead. A ray's positions do not
+// depend on what it reads, so a lane computes its next U voxels, requests
+// their U grid words together and then tests them in order: one fetch latency
+// per U steps instead of per step, for U - 1 fetches too many per ray. In a
+// launch that fills the chip those fetches are what binds (the ring above
+// fetches only where a ray enters another cell): trace_tile_waves draws the
+// line. Whole vx_trace calls before and after: 61x43 pixels of 64^3, 6 DDA
+// rays each, 124 -> 24 us; 320x180 of 512^3, 6 rays, 142 -> 41 us; 61x43 of
+// 512^3, 1 Sparse + 16 SuperSparse + 1, 275 -> 55 us (one thread per pixel).
+// ===========================================================================
+constexpr int kTileAhead = 4;      // voxels (DDA) per fetch latency
+constexpr int kTileSparse = 4;     // positions of a sparse march per fetch latency (2: 5-15 % slower)
+constexpr int kTileMaxWaves = 16;
+
+// Fast-path ray (fast_ray_ok, origin voxel cv inside the bounds) through the
+// march grid; true and its best_t when it hits. A voxel requested past the one
+// that ends the ray may lie outside the grid: its index is clamped to the last
+// word and what it reads is dropped (a ray cannot leave the grid without
+// meeting a border voxel, whose bit is set, first).
+template <int U>
+VXD bool dda_ahead(GridPtr grid, uint32_t gx, uint32_t gxy, uint32_t last, const int32_t lim[3], f3 o, f3 d,
+                   const int32_t cv[3], float maxt, float& t_hit) {
+    static_assert(256 % U == 0, "the step limit is tested at the end of a group");
+    const float oo[3] = {o.x, o.y, o.z}, dd[3] = {d.x, d.y, d.z};
+    float tm[3], td[3];
+    int32_t p[3], sp[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const bool neg = !(dd[k] > 0.0f);
+        const float nb = (float)cv[k] + (neg ? 0.0f : 1.0f);
+        tm[k] = (nb - oo[k]) / dd[k];
+        td[k] = 1.0f / (dd[k] * (neg ? -1.0f : 1.0f));
+        p[k] = (cv[k] + 4) << (2 * k);
+        sp[k] = (neg ? -1 : 1) * (1 << (2 * k));
+    }
+    for (int32_t n = 0; n < 256; n += U) {
+        uint64_t w[U];
+        uint32_t sh[U];
+        float bt[U];
+        const float t0[3] = {tm[0], tm[1], tm[2]};
+        const int32_t p0[3] = {p[0], p[1], p[2]};
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            sh[u] = cell_shift((uint32_t)p[0], (uint32_t)p[1], (uint32_t)p[2]);
+            w[u] = grid[min(grid_word(p[0], p[1], p[2], gx, gxy), last)];
+            const float t = fminf(fminf(tm[0], tm[1]), tm[2]);
+            bt[u] = best_t_of(tm[0], tm[1], tm[2]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const bool m = tm[k] == t;
+                p[k] += m ? sp[k] : 0;
+                tm[k] = m ? tm[k] + td[k] : tm[k];
+            }
+        }
+        int32_t end = U;
+        bool occ = false;
+#pragma unroll
+        for (int u = U - 1; u >= 0; --u) {
+            const bool b = (int64_t)(w[u] << (sh[u] & 63u)) < 0;
+            if (b || !(bt[u] < maxt)) {
+                end = u;
+                occ = b;
+                t_hit = bt[u];
+            }
+        }
+        if (end == U) continue;
+        if (!occ) return false;
+        // the voxel it stopped in: the group's first `end` steps again
+        int32_t q[3] = {p0[0], p0[1], p0[2]};
+        float tq[3] = {t0[0], t0[1], t0[2]};
+#pragma unroll
+        for (int u = 0; u < U - 1; ++u) {
+            if (u >= end) break;
+            const float t = fminf(fminf(tq[0], tq[1]), tq[2]);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const bool m = tq[k] == t;
+                q[k] += m ? sp[k] : 0;
+                tq[k] = m ? tq[k] + td[k] : tq[k];
+            }
+        }
+        return (uint32_t)(q[0] - 4) <= (uint32_t)lim[0] && (uint32_t)((q[1] >> 2) - 4) <= (uint32_t)lim[1] &&
+               (uint32_t)((q[2] >> 4) - 4) <= (uint32_t)lim[2];
+    }
+    return false;
+}
+
+// DDA / SPARSE: whether any ray class takes that marcher.
+template <bool DDA, bool SPARSE>
+__global__ void __launch_bounds__(64 * kTileMaxWaves) k_trace_tile(MarchArgs A) {
+    extern __shared__ float fold_s[];   // nrays x 64: 1 / 0 lit (shadow), min(t, maxt) / maxt (AO, spec)
+    __shared__ uint32_t next_s, done_s;
+    const MarchItem& I = A.item0;
+    const uint32_t lane = threadIdx.x & 63u, waves = blockDim.x >> 6;
+    // consecutive tiles on one XCD
+    const uint32_t lt = (blockIdx.x & 7u) * A.band_tiles + (blockIdx.x >> 3);
+    if (lt >= A.ntiles) return;   // block-uniform
+    if (threadIdx.x == 0) next_s = done_s = 0;
+    __syncthreads();
+    uint32_t i = 0;
+    const bool inview = tile_lane_pixel(I, lt, lane, i);
+    const TraceArgs& T = I.T;
+    const vx_trace_params& P = T.params;
+    const bool valid = inview && T.mat[i] != 0;
+    PixState S;
+    S.org = mk3(0.0f, 0.0f, 0.0f); S.pk = 0; S.i = 0;
+    f3 wd = mk3(0.0f, 0.0f, 0.0f);
+    if (valid) pixel_setup(T, i, S, wd);
+    const int32_t nlong = P.n_shadow + P.n_spec;
+    while (__ballot(valid) != 0) {
+        // shadow, spec, then AO rays
+        uint32_t g = 0;
+        if (lane == 0) g = atomicAdd(&next_s, 1u);
+        g = __builtin_amdgcn_readfirstlane(g);
+        if ((int32_t)g >= A.nrays) break;
+        const int32_t r = (int32_t)g < P.n_shadow ? (int32_t)g
+                          : ((int32_t)g < nlong ? A.nrays - 1 - ((int32_t)g - P.n_shadow) : (int32_t)g - P.n_spec);
+        if (!valid) continue;
+        f3 o, d;
+        float maxt;
+        const int32_t kind = pixel_ray(T, S, wd, r, o, d, maxt);
+        const int32_t march = kind == RAY_SHADOW ? P.shadow_march : (kind == RAY_AO ? P.ao_march : P.spec_march);
+        float v;
+        if (DDA && (!SPARSE || march == VX_MARCH_DDA)) {
+            bool hit = false;
+            float t = 0.0f;
+            if (fast_ray_ok(o, d)) {
+                int32_t cv[3];
+                ray_origin_voxel(o, cv);
+                if ((uint32_t)cv[0] <= (uint32_t)I.lim[0] && (uint32_t)cv[1] <= (uint32_t)I.lim[1] &&
+                    (uint32_t)cv[2] <= (uint32_t)I.lim[2])
+                    hit = dda_ahead<kTileAhead>(grid_ptr(I.grid), (uint32_t)I.gx, (uint32_t)I.gxy, A.last_word, I.lim, o, d,
+                                                cv, maxt, t);
+            } else {
+                RayOut R;
+                R.t = 0.0f;
+                dda_exact(I.V, o, d, maxt, R);
+                hit = R.hit != 0;
+                t = R.t;
+            }
+            v = ray_value(kind, hit ? 1 : 0, t, maxt);
+        } else {
+            uint32_t nf = 0;
+            int32_t h;
+            const float t = march_dist<kTileSparse>(I.V, march, o, d, maxt, nf, h);
+            v = kind == RAY_SHADOW ? (t != maxt ? 0.0f : 1.0f) : gmin(t, maxt) / maxt;
+        }
+        fold_s[(r << 6) + (int32_t)lane] = v;
+    }
+    if (waves > 1) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        uint32_t n = 0;
+        if (lane == 0) n = __hip_atomic_fetch_add(&done_s, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (__builtin_amdgcn_readfirstlane(n) != waves - 1u) return;
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    }
+    if (!inview) return;
+    if (!valid) {
+        T.shadow[i] = 0; T.ao[i] = 0.0f; T.spec[i] = 0.0f;
+        return;
+    }
+    // the pixel's rays in ray order (LightAmbient.frag:160-175)
+    float aosum = 0.0f;
+    for (int32_t a = 0; a < P.n_ao; ++a) {
+        const float q = fold_s[((P.n_shadow + a) << 6) + (int32_t)lane];
+        aosum = aosum + q * q;
+    }
+    T.shadow[i] = P.n_shadow > 0 ? (uint8_t)fold_s[lane] : 1;
+    T.ao[i] = P.n_ao > 0 ? aosum / (float)P.n_ao : 1.0f;
+    T.spec[i] = P.n_spec > 0 ? fold_s[((P.n_shadow + P.n_ao) << 6) + (int32_t)lane] : 1.0f;
+}
+
+// Waves per tile of k_trace_tile for a launch of ntiles tiles, 0 where another
+// kernel is the faster one. All-DDA rays: one wave per ray index while that is
+// at most two chips of waves (256 CUs x 32 waves); whole calls, tile against
+// ring: 16200 waves 136 / 162 us, 18000 waves 100 / 113 us (4 AO rays to 16) but
+// 43200 waves 307 / 207 us and 64800 waves 357 / 218 us. Sparse marchers: as
+// many waves as fill the chip once (more of them repeat a pixel's set-up: 640x360
+// with 1 + 4 rays 63 us at 2 waves per tile, 68 at 4, 75 at 5), and the
+// per-pixel kernel once one wave per tile does.
+uint32_t trace_tile_waves(uint32_t ntiles, int32_t nrays, bool all_dda) {
+    constexpr uint32_t kChipWaves = 8192;
+    if (nrays == 0) return 1;
+    const uint32_t most = std::min<uint32_t>((uint32_t)nrays, kTileMaxWaves);
+    if (all_dda) return (uint64_t)ntiles * (uint32_t)nrays > 2 * kChipWaves ? 0 : most;
+    const uint32_t fill = kChipWaves / ntiles;
+    return fill < std::min(most, 2u) ? 0 : std::min(fill, most);
+}
+
+hipError_t launch_trace_tile(bool dda, bool sparse, uint32_t waves, hipStream_t s, const MarchArgs& A) {
+    const dim3 grid(8 * A.band_tiles), block(64 * waves);
+    const size_t lds = std::max<size_t>((size_t)A.nrays * 64 * sizeof(float), 4);
+    if (dda && sparse) hipLaunchKernelGGL((k_trace_tile<true, true>), grid, block, lds, s, A);
+    else if (sparse) hipLaunchKernelGGL((k_trace_tile<false, true>), grid, block, lds, s, A);
+    else hipLaunchKernelGGL((k_trace_tile<true, false>), grid, block, lds, s, A);
+    return hipGetLastError();
 }
 
 // Launchers (template instances live in this file).
