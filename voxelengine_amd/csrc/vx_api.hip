@@ -555,13 +555,10 @@ extern "C" vx_status vx_model_download(const vx_model* m, int32_t mip, uint8_t* 
 extern "C" vx_status vx_model_build_mips(vx_model* m, void* stream) {
     VX_REQUIRE(m, "model is NULL");
     if (vx_status st = use_device(m->ctx)) return st;
-    for (int k = 1; k < 3; ++k) {
-        int32_t px = m->dims[0] >> (k - 1), py = m->dims[1] >> (k - 1), pz = m->dims[2] >> (k - 1);
-        size_t n = (size_t)(px / 2) * (py / 2) * (pz / 2);
-        hipLaunchKernelGGL(k_build_mip, dim3(cdiv(n, 256)), dim3(256), 0, S(stream), m->mip[k - 1], px, py, pz,
-                           m->mip[k]);
-        VX_LAUNCHED("k_build_mip");
-    }
+    const size_t n = (size_t)(m->dims[0] / 4) * (m->dims[1] / 4) * (m->dims[2] / 4);
+    hipLaunchKernelGGL(k_build_mips, dim3(cdiv(n, 256)), dim3(256), 0, S(stream), m->mip[0], m->dims[0], m->dims[1],
+                       m->dims[2], m->mip[1], m->mip[2]);
+    VX_LAUNCHED("k_build_mips");
     return VX_OK;
 }
 
@@ -679,13 +676,23 @@ extern "C" vx_status vx_volume_dims(const vx_volume* v, int32_t dims[3], int32_t
 extern "C" vx_status vx_volume_clear(vx_volume* v, void* stream) {
     VX_REQUIRE(v, "volume is NULL");
     if (vx_status st = use_device(v->ctx)) return st;
-    hipLaunchKernelGGL(k_fill_u64, dim3(cdiv(v->ncells, 256)), dim3(256), 0, S(stream), v->cells, v->ncells, 0ull);
-    for (int l = 0; l < v->nlevels; ++l) {
-        size_t nw = (size_t)v->wx[l] * v->wy[l] * v->wz[l];
-        hipLaunchKernelGGL(k_fill_u64, dim3(cdiv(nw, 256)), dim3(256), 0, S(stream), v->lvl[l], nw, 0ull);
+    ClearArgs A;
+    std::memset(&A, 0, sizeof(A));
+    uint64_t* p[4] = {v->cells, v->lvl[0], v->lvl[1], v->lvl[2]};
+    uint64_t blocks = 0;
+    for (int k = 0; k <= v->nlevels; ++k) {
+        A.p[k] = p[k];
+        A.words[k] = k == 0 ? v->ncells : (size_t)v->wx[k - 1] * v->wy[k - 1] * v->wz[k - 1];
+        A.blocks[k] = cdiv(A.words[k], 512);
+        blocks += A.blocks[k];
     }
-    VX_LAUNCHED("k_fill_u64");
-    if (hipError_t e = mgrid_full(v, S(stream))) return fail(VX_ERR_DEVICE, "march grid: %s", hipGetErrorString(e));
+    A.grid = v->grid;
+    A.ngrid = v->ngrid;
+    A.gx = v->gx;
+    A.gy = v->gy;
+    blocks += cdiv(v->ngrid, 256);
+    hipLaunchKernelGGL(k_clear_volume, dim3((uint32_t)blocks), dim3(256), 0, S(stream), A, occ_view(v));
+    VX_LAUNCHED("k_clear_volume");
     return VX_OK;
 }
 
@@ -774,6 +781,7 @@ static PlannedOp make_op(const vx_instance& in, const float m[16], int32_t value
         o.dy[k] = m[4 + k] * 0.1f;
         o.dz[k] = m[8 + k] * 0.1f;
     }
+    o.axis = o.dx[1] == 0.0f && o.dx[2] == 0.0f && o.dy[0] == 0.0f && o.dy[2] == 0.0f && o.dz[0] == 0.0f && o.dz[1] == 0.0f;
     // Corners of the voxel index box mapped exactly, widened by two fine
     // voxels for fp32 rounding and truncation.
     for (int k = 0; k < 3; ++k) {
@@ -831,10 +839,13 @@ static vx_status vx_volume_rebuild_impl(vx_volume* v, const vx_instance* inst, u
         } else {
             float np[3] = {-in.pivot[0], -in.pivot[1], -in.pivot[2]};
             float m[16];
+            float c[16];
             translate(in.prev, np, m);
-            ops.push_back(make_op(in, m, 0, (int32_t)i));
-            translate(in.cur, np, m);
-            ops.push_back(make_op(in, m, 1, (int32_t)i));
+            translate(in.cur, np, c);
+            // An instance that has not moved erases exactly the voxels that its
+            // write sets next: the write alone leaves the same volume and AABB.
+            if (std::memcmp(m, c, sizeof(m)) != 0) ops.push_back(make_op(in, m, 0, (int32_t)i));
+            ops.push_back(make_op(in, c, 1, (int32_t)i));
         }
     }
     std::vector<std::vector<int>> batches;
@@ -898,10 +909,12 @@ static vx_status vx_volume_rebuild_impl(vx_volume* v, const vx_instance* inst, u
         e = hipMemcpyAsync(ops_d, flat.data(), flat.size() * sizeof(FootprintOp), hipMemcpyHostToDevice, S(stream));
     OccView V = occ_view(v);
     for (size_t b = 0; b < batches.size() && e == hipSuccess; ++b) {
-        size_t maxq = 0;   // quads of four x voxels
-        for (int q : batches[b])
-            maxq = std::max(maxq, (size_t)((ops[q].op.sx + 3) / 4) * ops[q].op.sy * ops[q].op.sz);
-        uint32_t gx = std::min<uint32_t>(cdiv(maxq, 256), 4096);
+        size_t maxu = 0;   // a thread's blocks of model voxels (k_footprint)
+        for (int q : batches[b]) {
+            const FootprintOp& o = ops[q].op;
+            maxu = std::max(maxu, (size_t)((o.sx + 3) / 4) * ((o.sy + 3) / 4) * (o.axis ? (o.sz + 3) / 4 : o.sz));
+        }
+        uint32_t gx = (uint32_t)std::min<size_t>((maxu + 255) / 256, 2048);
         for (size_t c0 = 0; c0 < batches[b].size() && e == hipSuccess; c0 += 65535) {
             uint32_t cnt = (uint32_t)std::min<size_t>(65535, batches[b].size() - c0);
             hipLaunchKernelGGL(k_footprint, dim3(gx, cnt), dim3(256), 0, S(stream), v->cells, V,
@@ -1005,22 +1018,33 @@ static vx_status vx_volume_build_levels_impl(vx_volume* v, const vx_region* regi
         }
     }
     OccView V = occ_view(v);
-    for (auto& br : ranges) {
-        for (int l = 0; l < v->nlevels; ++l) {
-            // level l+1 words covering the brick range: word = brick >> (3l + 2)
-            int32_t sh = 3 * l + 2;
-            int32_t w0[3], w1[3];
-            for (int k = 0; k < 3; ++k) { w0[k] = br[k] >> sh; w1[k] = br[3 + k] >> sh; }
-            int32_t nw[3] = {w1[0] - w0[0] + 1, w1[1] - w0[1] + 1, w1[2] - w0[2] + 1};
-            size_t nthreads = (size_t)nw[0] * nw[1] * nw[2] * 64;
-            if (l == 0) {
-                hipLaunchKernelGGL(k_level1, dim3(cdiv(nthreads, 256)), dim3(256), 0, S(stream), v->lvl[0], v->cells,
-                                   V, w0[0], w0[1], w0[2], nw[0], nw[1], nw[2]);
-            } else {
-                hipLaunchKernelGGL(k_level_up, dim3(cdiv(nthreads, 256)), dim3(256), 0, S(stream), v->lvl[l],
-                                   v->lvl[l - 1], v->wx[l - 1], v->wy[l - 1], v->wz[l - 1], v->wx[l], v->wy[l],
-                                   v->wz[l], w0[0], w0[1], w0[2], nw[0], nw[1], nw[2]);
+    // level by level (a level reads the one below), up to kLevelRanges ranges per launch
+    for (int l = 0; l < v->nlevels; ++l) {
+        // level l+1 words covering a brick range: word = brick >> (3l + 2)
+        const int32_t sh = 3 * l + 2;
+        for (size_t r0 = 0; r0 < ranges.size(); r0 += kLevelRanges) {
+            const uint32_t cnt = (uint32_t)std::min<size_t>(kLevelRanges, ranges.size() - r0);
+            LevelRanges R;
+            std::memset(&R, 0, sizeof(R));
+            uint32_t blocks = 0;
+            R.n = cnt;
+            for (uint32_t i = 0; i < cnt; ++i) {
+                const std::array<int32_t, 6>& br = ranges[r0 + i];
+                size_t words = 1;
+                for (int k = 0; k < 3; ++k) {
+                    R.r[i][k] = (uint16_t)(br[k] >> sh);
+                    R.r[i][3 + k] = (uint16_t)((br[3 + k] >> sh) - (br[k] >> sh) + 1);
+                    words *= R.r[i][3 + k];
+                }
+                R.block0[i] = blocks;
+                blocks += cdiv(words, 4);
             }
+            const dim3 grid(blocks);
+            if (l == 0)
+                hipLaunchKernelGGL(k_level1, grid, dim3(256), 0, S(stream), v->lvl[0], v->cells, V, R);
+            else
+                hipLaunchKernelGGL(k_level_up, grid, dim3(256), 0, S(stream), v->lvl[l], v->lvl[l - 1], v->wx[l - 1],
+                                   v->wy[l - 1], v->wz[l - 1], v->wx[l], v->wy[l], R);
             VX_LAUNCHED("level build");
         }
     }
@@ -1227,7 +1251,7 @@ static vx_status vx_primary_instances_impl(vx_ctx* ctx, const vx_vox_cmd* cmds, 
     B.ntiles = tiles.ntiles;
     B.lists = ctx->tile_lists;
     B.counts = ctx->tile_counts;
-    hipLaunchKernelGGL(k_bin_instances, dim3(cdiv(tiles.ntiles, 256)), dim3(256), 0, S(stream), B);
+    hipLaunchKernelGGL(k_bin_instances, dim3(cdiv(tiles.ntiles, 4)), dim3(256), 0, S(stream), B);
     VX_LAUNCHED("k_bin_instances");
     PrimaryInstArgs A;
     A.view = *view;

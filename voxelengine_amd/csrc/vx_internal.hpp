@@ -13,7 +13,27 @@ struct FootprintOp {
     int32_t sx, sy, sz;
     int32_t value;     // 0 erase, 1 write
     int32_t inst;      // instance slot for the dirty AABB
+    int32_t axis;      // coordinate k depends on model axis k only (dx, dy, dz diagonal)
     float o[3], dx[3], dy[3], dz[3];
+};
+
+// Word ranges of one coarse-level launch: first word and word count per axis
+// (a volume of 4096 texels per axis has 257 level-1 words per axis).
+constexpr uint32_t kLevelRanges = 128;
+struct LevelRanges {
+    uint32_t n;                        // ranges of this launch
+    uint32_t block0[kLevelRanges];     // each range's first block (four words per block)
+    uint16_t r[kLevelRanges][6];
+};
+
+// The arrays of a volume (cells, levels 1..3, march grid) to be emptied.
+struct ClearArgs {
+    uint64_t* p[4];
+    size_t words[4];
+    uint32_t blocks[4];                // 512 words each
+    uint64_t* grid;
+    size_t ngrid;
+    int32_t gx, gy;
 };
 
 // Block -> pixel tile mapping (16x16 pixels per 256-thread block).
@@ -244,17 +264,18 @@ __global__ void k_terrain_fill(uint8_t* vol, const float* h, int32_t nx, int32_t
                                int32_t use_terrain);
 __global__ void k_boxes(uint8_t* vol, int32_t nx, int32_t ny, int32_t nz, uint32_t seed, int32_t b0, int32_t emin,
                         int32_t emax, int32_t grounded);
-__global__ void k_build_mip(const uint8_t* parent, int32_t px, int32_t py, int32_t pz, uint8_t* out);
+__global__ void __launch_bounds__(256) k_build_mips(const uint8_t* m0, int32_t px, int32_t py, int32_t pz, uint8_t* m1,
+                                                    uint8_t* m2);
 __global__ void k_fill_u64(uint64_t* p, size_t n, uint64_t v);
 __global__ void k_bytes_to_cells(uint64_t* cells, const uint8_t* bytes, OccView V, int32_t rx, int32_t ry, int32_t rz,
                                  int32_t rw, int32_t rh, int32_t rd);
 __global__ void k_cells_to_bytes(uint8_t* bytes, const uint64_t* cells, OccView V);
-__global__ void k_footprint(uint64_t* cells, OccView V, const FootprintOp* ops, int32_t* aabb, int32_t thr);
-__global__ void k_level1(uint64_t* words, const uint64_t* cells, OccView V, int32_t w0x, int32_t w0y, int32_t w0z,
-                         int32_t nwx, int32_t nwy, int32_t nwz);
-__global__ void k_level_up(uint64_t* words, const uint64_t* lower, int32_t lwx, int32_t lwy, int32_t lwz, int32_t uwx,
-                           int32_t uwy, int32_t uwz, int32_t w0x, int32_t w0y, int32_t w0z, int32_t nwx, int32_t nwy,
-                           int32_t nwz);
+__global__ void __launch_bounds__(256) k_footprint(uint64_t* cells, OccView V, const FootprintOp* ops, int32_t* aabb,
+                                                   int32_t thr);
+__global__ void __launch_bounds__(256) k_level1(uint64_t* words, const uint64_t* cells, OccView V, LevelRanges R);
+__global__ void __launch_bounds__(256) k_level_up(uint64_t* words, const uint64_t* lower, int32_t lwx, int32_t lwy,
+                                                  int32_t lwz, int32_t uwx, int32_t uwy, LevelRanges R);
+__global__ void __launch_bounds__(256) k_clear_volume(ClearArgs A, OccView V);
 __global__ void k_trace_rays(OccView V, const float* rays, uint32_t n, int32_t march, vx_ray_result* out);
 __global__ void __launch_bounds__(256) k_trace(OccView V, TraceArgs A);
 __global__ void k_zero_u32(uint32_t* p, int n);
@@ -278,8 +299,8 @@ __global__ void __launch_bounds__(256) k_shade_bwd_batch(const ShadeArgs* items,
 __global__ void k_shade_bwd_finish(const long long* acc, float* dpal, float* dlight);
 __global__ void k_zero_i64(long long* p, int n);
 
-__global__ void k_mgrid(uint64_t* grid, OccView V, int32_t gx, int32_t gy, int32_t g0x, int32_t g0y, int32_t g0z,
-                        int32_t nx, int32_t ny, int32_t nz);
+__global__ void __launch_bounds__(256) k_mgrid(uint64_t* grid, OccView V, int32_t gx, int32_t gy, int32_t g0x, int32_t g0y,
+                                               int32_t g0z, int32_t nx, int32_t ny, int32_t nz);
 
 // Ray-parallel trace, instantiated for 256/512-thread blocks and 2/4/8 DDA
 // steps between refills; launch_march enqueues march, listed rays and resolve
