@@ -310,13 +310,23 @@ static OccView occ_view(const vx_volume* v) {
     return V;
 }
 
+// Length of an XCD's runs of tiles (log2): at most 16 tiles, at least eight runs
+// per XCD. Runs of 1, 4, 16 and 64: lights 611 / 614 / 602 / 618 us at 1080p,
+// primary 445 / 438 / 442 / 450 us.
+static uint32_t tile_run_shift(uint32_t ntiles) {
+    uint32_t s = 0;
+    while (s < 4 && ntiles >= (128u << s)) ++s;
+    return s;
+}
+
 static TileMap tile_map(int32_t w, int32_t h) {
     TileMap t;
     t.width = w;
     t.height = h;
     t.tiles_x = cdiv((uint32_t)w, 16);
     t.ntiles = t.tiles_x * cdiv((uint32_t)h, 16);
-    t.per_xcd = cdiv(t.ntiles, 8);
+    t.run_shift = tile_run_shift(t.ntiles);
+    t.blocks = cdiv(t.ntiles, 8u << t.run_shift) * (8u << t.run_shift);
     return t;
 }
 
@@ -1088,7 +1098,7 @@ extern "C" vx_status vx_primary(vx_ctx* ctx, const vx_model* model, const vx_vie
     mat_mul_f32(view->proj, view->view, A.pv);
     for (int k = 0; k < 3; ++k) { A.mips[k] = model->mip[k]; A.dims[k] = model->dims[k]; }
     A.pos = g->pos; A.nrm = g->normal; A.mat = g->material;
-    hipLaunchKernelGGL(k_primary, dim3(8 * A.tiles.per_xcd), dim3(256), 0, S(stream), A);
+    hipLaunchKernelGGL(k_primary, dim3(A.tiles.blocks), dim3(256), 0, S(stream), A);
     VX_LAUNCHED("k_primary");
     return VX_OK;
 }
@@ -1266,7 +1276,7 @@ static vx_status vx_primary_instances_impl(vx_ctx* ctx, const vx_vox_cmd* cmds, 
     A.motion = ext ? ext->motion : nullptr;
     A.depth = ext ? ext->depth : nullptr;
     A.palette = ext ? ext->palette : nullptr;
-    hipLaunchKernelGGL(k_primary_inst, dim3(8 * tiles.per_xcd), dim3(256), 0, S(stream), A);
+    hipLaunchKernelGGL(k_primary_inst, dim3(tiles.blocks), dim3(256), 0, S(stream), A);
     VX_LAUNCHED("k_primary_inst");
     return VX_OK;
 }
@@ -1522,7 +1532,7 @@ static vx_status launch_trace_tile_view(vx_ctx* ctx, const vx_volume* vol, const
     A.item0 = make_march_item(vol, T, 0u, g);
     A.nrays = T.params.n_shadow + T.params.n_ao + T.params.n_spec;
     A.ntiles = g.ntiles;
-    A.band_tiles = cdiv(g.ntiles, 8);
+    A.run_shift = tile_run_shift(g.ntiles);
     A.last_word = (uint32_t)(vol->ngrid - 1);
     const vx_trace_params& p = T.params;
     const int32_t n[3] = {p.n_shadow, p.n_ao, p.n_spec}, m[3] = {p.shadow_march, p.ao_march, p.spec_march};
@@ -1592,7 +1602,7 @@ static vx_status trace_impl(vx_ctx* ctx, const vx_volume* vol, const vx_view* vi
     }
     if (all_dda && ctx->tuning.kernel != 1)
         return noalloc ? launch_trace_march_noalloc(ctx, vol, A, S(stream)) : launch_trace_march(ctx, vol, A, S(stream));
-    hipLaunchKernelGGL(k_trace, dim3(8 * A.tiles.per_xcd), dim3(256), 0, S(stream), occ_view(vol), A);
+    hipLaunchKernelGGL(k_trace, dim3(A.tiles.blocks), dim3(256), 0, S(stream), occ_view(vol), A);
     VX_LAUNCHED("k_trace");
     return VX_OK;
 }
@@ -1664,7 +1674,7 @@ static vx_status light_pass_list(vx_ctx* ctx, const vx_volume* vol, const LightA
     B.slot_light = nullptr;
     B.rfetch = nullptr;
     hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, stream, B.total, 1);
-    hipLaunchKernelGGL(k_light_count, dim3(8 * A.tiles.per_xcd), dim3(256), 0, stream, A, B);
+    hipLaunchKernelGGL(k_light_count, dim3(A.tiles.blocks), dim3(256), 0, stream, A, B);
     VX_LAUNCHED("k_light_count");
     uint32_t total = 0;
     VX_HIP(hipMemcpyAsync(&total, B.total, sizeof(uint32_t), hipMemcpyDeviceToHost, stream));
@@ -1688,7 +1698,7 @@ static vx_status light_pass_list(vx_ctx* ctx, const vx_volume* vol, const LightA
     B.shadow = ctx->lt_shadow;
     B.slot_light = ctx->lt_slot_light;
     B.rfetch = A.fetches ? ctx->lt_rfetch : nullptr;
-    hipLaunchKernelGGL(k_light_records, dim3(8 * A.tiles.per_xcd), dim3(256), 0, stream, A, B);
+    hipLaunchKernelGGL(k_light_records, dim3(A.tiles.blocks), dim3(256), 0, stream, A, B);
     VX_LAUNCHED("k_light_records");
     const uint32_t grid = std::min<uint32_t>(cdiv(total, 256), (uint32_t)ctx->gcache.cus * 8u);
     hipLaunchKernelGGL(k_light_march, dim3(grid), dim3(256), 0, stream, occ_view(vol), A, B);
@@ -1720,7 +1730,7 @@ extern "C" vx_status vx_light_pass(vx_ctx* ctx, const vx_volume* vol, const vx_v
     A.rgb = rgb;
     A.fetches = fetches;
     if (ctx->tuning.lights == 0 || nlights == 0) {
-        hipLaunchKernelGGL(k_lights, dim3(8 * A.tiles.per_xcd), dim3(256), 0, S(stream), occ_view(vol), A);
+        hipLaunchKernelGGL(k_lights, dim3(A.tiles.blocks), dim3(256), 0, S(stream), occ_view(vol), A);
         VX_LAUNCHED("k_lights");
         return VX_OK;
     }
@@ -1754,7 +1764,7 @@ extern "C" vx_status vx_reflection(vx_ctx* ctx, const vx_volume* vol, const vx_v
     A.params = *params;
     A.out = io->out;
     A.t = io->t;
-    hipLaunchKernelGGL(k_reflection, dim3(8 * A.tiles.per_xcd), dim3(256), 0, S(stream), occ_view(vol), A);
+    hipLaunchKernelGGL(k_reflection, dim3(A.tiles.blocks), dim3(256), 0, S(stream), occ_view(vol), A);
     VX_LAUNCHED("k_reflection");
     return VX_OK;
 }

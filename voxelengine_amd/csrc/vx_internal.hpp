@@ -36,10 +36,12 @@ struct ClearArgs {
     int32_t gx, gy;
 };
 
-// Block -> pixel tile mapping (16x16 pixels per 256-thread block).
+// Block -> pixel tile mapping (16x16 pixels per 256-thread block; tile_of_block).
 struct TileMap {
     int32_t width, height;
-    uint32_t tiles_x, ntiles, per_xcd;
+    uint32_t tiles_x, ntiles;
+    uint32_t run_shift;        // an XCD takes runs of 1 << run_shift tiles in turn
+    uint32_t blocks;           // blocks to launch
 };
 
 struct TraceArgs {
@@ -98,6 +100,7 @@ struct MarchArgs {
     int32_t refill;            // not-running lanes that trigger a refill
     float maxt[3];             // shadow, AO, spec
     uint32_t last_word;        // index of the march grid's last word (k_trace_tile)
+    uint32_t run_shift;        // k_trace_tile: an XCD's runs of 1 << run_shift tiles
 };
 
 struct LightArgs {
