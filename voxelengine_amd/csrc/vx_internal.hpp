@@ -233,7 +233,9 @@ struct TaaArgs {
     const uint8_t* mat;       // material index per pixel
     const float* palette;     // 256 x 6
     float* out;               // 4 per pixel
-    float4* rec;              // 4 float4 per pixel: packed attributes (k_taa_pack)
+    TileMap tiles;
+    uint64_t* off;            // per tile and wave: the pixels whose history lies off the image
+    int32_t tile_waves;       // waves per tile
 };
 
 struct PrimaryArgs {
@@ -293,8 +295,10 @@ __global__ void __launch_bounds__(256) k_gbuf_depth(DepthArgs A);
 __global__ void __launch_bounds__(256) k_ssao(SsaoArgs A);
 __global__ void __launch_bounds__(256) k_bin_instances(BinArgs A);
 __global__ void __launch_bounds__(256) k_primary_inst(PrimaryInstArgs A);
-__global__ void __launch_bounds__(256) k_taa_pack(TaaArgs A);
-__global__ void __launch_bounds__(256) k_light_taa(TaaArgs A);
+__global__ void __launch_bounds__(1024) k_light_taa32(TaaArgs A);
+__global__ void __launch_bounds__(256) k_light_taa16(TaaArgs A);
+__global__ void __launch_bounds__(1024) k_light_taa_off(TaaArgs A);
+__global__ void __launch_bounds__(256) k_copy_f32(float* dst, const float* src, size_t n);
 __global__ void k_shade_fwd(ShadeArgs A);
 __global__ void __launch_bounds__(256) k_shade_bwd(ShadeArgs A, long long* acc);
 __global__ void __launch_bounds__(256) k_shade_bwd_batch(const ShadeArgs* items, const uint32_t* block0, uint32_t n,

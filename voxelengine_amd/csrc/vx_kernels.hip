@@ -2880,30 +2880,26 @@ __global__ void __launch_bounds__(256) k_primary_inst(PrimaryInstArgs A) {
 // index (the G-buffer colour / material attachments).
 // ===========================================================================
 namespace taa {
-// One pixel's attributes in one 64-byte record, so a bilinear sample of every
-// attribute loads four records (k_taa_pack writes them):
-//   v0 = light rgb, light alpha (1 on sky pixels)   v1 = colour rgb, depth
-//   v2 = material rgb, motion x                      v3 = normal xyz, motion y
-// The material's fourth channel is 0 inside the image and 1 on the border.
-struct Texel {
-    float4 v0, v1, v2, v3;
-};
+// Material code of a texel outside the image; the palette copy's entry for it
+// (and for 0, the sky) is zero.
+constexpr uint32_t kBorder = 256u;
 
-VXD Texel border_texel() {
-    Texel t;
-    t.v0 = make_float4(0.0f, 0.0f, 0.0f, 1.0f);
-    t.v1 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    t.v2 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    t.v3 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    return t;
+// Texel (x, y) from the G-buffer: light rgb and material code, normal and
+// depth, motion; the border reads zeros.
+VXD float4 light_at(const TaaArgs& A, int32_t x, int32_t y) {
+    if (x < 0 || y < 0 || x >= A.width || y >= A.height) return make_float4(0.0f, 0.0f, 0.0f, __uint_as_float(kBorder));
+    const size_t i = (size_t)y * A.width + x;
+    return make_float4(A.light[3 * i], A.light[3 * i + 1], A.light[3 * i + 2], __uint_as_float((uint32_t)A.mat[i]));
 }
-
-VXD Texel fetch(const TaaArgs& A, int32_t x, int32_t y) {
-    if (x < 0 || y < 0 || x >= A.width || y >= A.height) return border_texel();
-    const float4* r = A.rec + 4 * ((size_t)y * A.width + x);
-    Texel t;
-    t.v0 = r[0]; t.v1 = r[1]; t.v2 = r[2]; t.v3 = r[3];
-    return t;
+VXD float4 normal_at(const TaaArgs& A, int32_t x, int32_t y) {
+    if (x < 0 || y < 0 || x >= A.width || y >= A.height) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const size_t i = (size_t)y * A.width + x;
+    return make_float4(A.normal[3 * i], A.normal[3 * i + 1], A.normal[3 * i + 2], A.depth[i]);
+}
+VXD float2 motion_at(const TaaArgs& A, int32_t x, int32_t y) {
+    if (!A.motion || x < 0 || y < 0 || x >= A.width || y >= A.height) return make_float2(0.0f, 0.0f);
+    const size_t i = (size_t)y * A.width + x;
+    return make_float2(A.motion[2 * i], A.motion[2 * i + 1]);
 }
 
 // Sub-texel weight: the fraction rounded to 1/256; 1 moves to the next texel.
@@ -2925,36 +2921,98 @@ VXD float bl(float a, float b, float c, float d, float fx, float fy) {
     return (a * (1.0f - fx) + b * fx) * (1.0f - fy) + (c * (1.0f - fx) + d * fx) * fy;
 }
 
-// Every attribute of texture(*, uv).
-struct Sample {
-    float light[4], color[3], depth, matl[4], nrm[3], mo[2];
+// An image tile of T x T pixels with its neighbourhood in LDS: a spiral sample
+// lies within 13 * (variance + 1) * 0.5 pixels, 13 for the variance's range of
+// [0, 1], a neighbour of an off-screen pixel (8-pixel tiles) within 9, and its
+// bilinear texels one further on the right and below.
+template <int T>
+struct Tile {
+    static constexpr int kHalo = T == 8 ? 9 : 13, kEdge = T + 2 * kHalo + 1;
+    float4 lm[kEdge * kEdge];   // light rgb, material code
+    float4 nd[kEdge * kEdge];   // normal, depth
+    float2 mo[kEdge * kEdge];   // motion
+    float pal[(kBorder + 1) * 6];
 };
 
-VXD void sample_all(const TaaArgs& A, float u, float v, Sample& s) {
-    int32_t x0, y0;
+// A bilinear sample position: its first texel, weights, and that texel's place
+// in the tile (in = all four texels lie there).
+struct Tap {
+    int32_t x0, y0, at;
     float fx, fy;
-    weight(u * (float)A.width - 0.5f, A.width, x0, fx);
-    weight(v * (float)A.height - 0.5f, A.height, y0, fy);
-    const Texel a = fetch(A, x0, y0), b = fetch(A, x0 + 1, y0), c = fetch(A, x0, y0 + 1), d = fetch(A, x0 + 1, y0 + 1);
-    s.light[0] = bl(a.v0.x, b.v0.x, c.v0.x, d.v0.x, fx, fy);
-    s.light[1] = bl(a.v0.y, b.v0.y, c.v0.y, d.v0.y, fx, fy);
-    s.light[2] = bl(a.v0.z, b.v0.z, c.v0.z, d.v0.z, fx, fy);
-    s.light[3] = bl(a.v0.w, b.v0.w, c.v0.w, d.v0.w, fx, fy);
-    s.color[0] = bl(a.v1.x, b.v1.x, c.v1.x, d.v1.x, fx, fy);
-    s.color[1] = bl(a.v1.y, b.v1.y, c.v1.y, d.v1.y, fx, fy);
-    s.color[2] = bl(a.v1.z, b.v1.z, c.v1.z, d.v1.z, fx, fy);
-    s.depth = bl(a.v1.w, b.v1.w, c.v1.w, d.v1.w, fx, fy);
-    s.matl[0] = bl(a.v2.x, b.v2.x, c.v2.x, d.v2.x, fx, fy);
-    s.matl[1] = bl(a.v2.y, b.v2.y, c.v2.y, d.v2.y, fx, fy);
-    s.matl[2] = bl(a.v2.z, b.v2.z, c.v2.z, d.v2.z, fx, fy);
-    const auto out = [&](int32_t x, int32_t y) { return (x < 0 || y < 0 || x >= A.width || y >= A.height) ? 1.0f : 0.0f; };
-    s.matl[3] = bl(out(x0, y0), out(x0 + 1, y0), out(x0, y0 + 1), out(x0 + 1, y0 + 1), fx, fy);
-    s.mo[0] = bl(a.v2.w, b.v2.w, c.v2.w, d.v2.w, fx, fy);
-    s.nrm[0] = bl(a.v3.x, b.v3.x, c.v3.x, d.v3.x, fx, fy);
-    s.nrm[1] = bl(a.v3.y, b.v3.y, c.v3.y, d.v3.y, fx, fy);
-    s.nrm[2] = bl(a.v3.z, b.v3.z, c.v3.z, d.v3.z, fx, fy);
-    s.mo[1] = bl(a.v3.w, b.v3.w, c.v3.w, d.v3.w, fx, fy);
-}
+    bool in;
+};
+
+template <int T>
+struct Sampler {
+    const TaaArgs& A;
+    const Tile<T>& L;
+    int32_t ox, oy;   // the tile's first texel
+    bool staged;      // the tile is loaded
+    bool skip;        // and holds no value that a zero weight may not cancel
+
+    VXD Tap tap(float u, float v) const {
+        Tap t;
+        weight(u * (float)A.width - 0.5f, A.width, t.x0, t.fx);
+        weight(v * (float)A.height - 0.5f, A.height, t.y0, t.fy);
+        const int32_t lx = t.x0 - ox, ly = t.y0 - oy;
+        t.in = staged && (uint32_t)lx < (uint32_t)(Tile<T>::kEdge - 1) && (uint32_t)ly < (uint32_t)(Tile<T>::kEdge - 1);
+        t.at = ly * Tile<T>::kEdge + lx;
+        return t;
+    }
+    template <class V, class G>
+    VXD void four(const Tap& t, const V* tile, G global, V q[4]) const {
+        if (t.in) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = tile[t.at + (k & 1) + (k >> 1) * Tile<T>::kEdge];
+        } else {
+#pragma unroll
+            for (int k = 0; k < 4; ++k) q[k] = global(A, t.x0 + (k & 1), t.y0 + (k >> 1));
+        }
+    }
+    VXD void light(const Tap& t, float rgb[3], uint32_t m[4]) const {
+        float4 q[4];
+        four(t, L.lm, light_at, q);
+        rgb[0] = bl(q[0].x, q[1].x, q[2].x, q[3].x, t.fx, t.fy);
+        rgb[1] = bl(q[0].y, q[1].y, q[2].y, q[3].y, t.fx, t.fy);
+        rgb[2] = bl(q[0].z, q[1].z, q[2].z, q[3].z, t.fx, t.fy);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) m[k] = __float_as_uint(q[k].w);
+    }
+    VXD void normal_depth(const Tap& t, float n[3], float& d) const {
+        float4 q[4];
+        four(t, L.nd, normal_at, q);
+        n[0] = bl(q[0].x, q[1].x, q[2].x, q[3].x, t.fx, t.fy);
+        n[1] = bl(q[0].y, q[1].y, q[2].y, q[3].y, t.fx, t.fy);
+        n[2] = bl(q[0].z, q[1].z, q[2].z, q[3].z, t.fx, t.fy);
+        d = bl(q[0].w, q[1].w, q[2].w, q[3].w, t.fx, t.fy);
+    }
+    VXD void motion(const Tap& t, float mo[2]) const {
+        float2 q[4];
+        four(t, L.mo, motion_at, q);
+        mo[0] = bl(q[0].x, q[1].x, q[2].x, q[3].x, t.fx, t.fy);
+        mo[1] = bl(q[0].y, q[1].y, q[2].y, q[3].y, t.fx, t.fy);
+    }
+    // Colour and material (its fourth channel is 1 on the border, 0 inside).
+    VXD void surface(const Tap& t, const uint32_t m[4], float s[7]) const {
+        if (m[0] == m[1] && m[0] == m[2] && m[0] == m[3]) {   // bl of one value, its two halves equal
+            const float* e = L.pal + 6 * m[0];
+#pragma unroll
+            for (int c = 0; c < 7; ++c) {
+                const float a = c < 6 ? e[c] : (m[0] == kBorder ? 1.0f : 0.0f);
+                const float r = a * (1.0f - t.fx) + a * t.fx;
+                s[c] = r * (1.0f - t.fy) + r * t.fy;
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < 6; ++c)
+                s[c] = bl(L.pal[6 * m[0] + c], L.pal[6 * m[1] + c], L.pal[6 * m[2] + c], L.pal[6 * m[3] + c], t.fx, t.fy);
+            float b[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) b[k] = m[k] == kBorder ? 1.0f : 0.0f;
+            s[6] = bl(b[0], b[1], b[2], b[3], t.fx, t.fy);
+        }
+    }
+};
 
 // texture(LAST_LIGHT_TEXTURE, uv): 4 channels, border (0, 0, 0, 1).
 VXD void sample_last(const TaaArgs& A, float u, float v, float* o) {
@@ -2977,77 +3035,111 @@ VXD void sample_last(const TaaArgs& A, float u, float v, float* o) {
 
 VXD float len2(float x, float y) { return sqrtf(x * x + y * y); }
 VXD float len3(float x, float y, float z) { return sqrtf((x * x + y * y) + z * z); }
-VXD float len4(const float* a, const float* b) {
-    const float d0 = a[0] - b[0], d1 = a[1] - b[1], d2 = a[2] - b[2], d3 = a[3] - b[3];
-    return sqrtf(((d0 * d0 + d1 * d1) + d2 * d2) + d3 * d3);
-}
-}  // namespace taa
 
-// One record per pixel from the G-buffer, the palette and this frame's light.
-__global__ void __launch_bounds__(256) k_taa_pack(TaaArgs A) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint32_t)(A.width * A.height)) return;
-    const uint32_t m = A.mat[i];
-    const float* pe = A.palette + 6 * m;
-    const float mx = A.motion ? A.motion[2 * (size_t)i] : 0.0f, my = A.motion ? A.motion[2 * (size_t)i + 1] : 0.0f;
-    float4* r = A.rec + 4 * (size_t)i;
-    r[0] = make_float4(A.light[3 * (size_t)i], A.light[3 * (size_t)i + 1], A.light[3 * (size_t)i + 2],
-                       m == 0 ? 1.0f : 0.0f);
-    r[1] = make_float4(m ? pe[0] : 0.0f, m ? pe[1] : 0.0f, m ? pe[2] : 0.0f, A.depth[i]);
-    r[2] = make_float4(m ? pe[3] : 0.0f, m ? pe[4] : 0.0f, m ? pe[5] : 0.0f, mx);
-    r[3] = make_float4(A.normal[3 * (size_t)i], A.normal[3 * (size_t)i + 1], A.normal[3 * (size_t)i + 2], my);
-}
+// Comparisons of a correctly rounded root as comparisons of its square, exact:
+// each is the largest float on its side.
+//   1 - sqrt(q) >= 0.8 as q <= kSameMaterial;  sqrt(q) <= 0.1 as q <= kSameMotion;
+//   sqrt(q) * 10000 < 1 as q <= kNearColor;    sqrt(q) < 1 as q <= kNearColorWide
+constexpr uint32_t kSameMaterial = 0x3d23d70bu, kSameMotion = 0x3c23d70bu, kNearColor = 0x322bcc75u, kNearColorWide = 0x3f7fffffu;
 
-__global__ void __launch_bounds__(256) k_light_taa(TaaArgs A) {
-    using namespace taa;
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (uint32_t)(A.width * A.height)) return;
-    const int32_t px = (int32_t)(i % (uint32_t)A.width), py = (int32_t)(i / (uint32_t)A.width);
-    const float W = (float)A.width, H = (float)A.height;
-    const float u = ((float)px + 0.5f) / W, v = ((float)py + 0.5f) / H;
-    const float irx = 1.0f / W, iry = 1.0f / H;
-    Sample c;
-    sample_all(A, u, v, c);
-    const float ou = u + c.mo[0], ov = v + c.mo[1];
-    float* o = A.out + 4 * (size_t)i;
-    if (c.depth == 1.0f) {
-        o[0] = c.light[0]; o[1] = c.light[1]; o[2] = c.light[2]; o[3] = c.light[3];
-        return;
+// The centre pixel's attributes.
+struct Centre {
+    float light[3], surf[7], nrm[3], depth, mo[2];
+};
+// A neighbour's light and its weight factors.
+struct Near {
+    float light[3], step, dot, depth, color;
+};
+
+// The neighbour at (u, v). With S.skip, a neighbour of another surface is left
+// at its light (false): a factor that is 0 makes the weight 0 when the others
+// are finite, and weight 0 adds nothing where the light is finite. far: the
+// motion differs by more than 0.1.
+template <int T, bool WIDE>
+VXD bool neighbour(const Sampler<T>& S, const Centre& c, float u, float v, Near& n, bool& far) {
+    const Tap t = S.tap(u, v);
+    uint32_t m[4];
+    float s[7];
+    S.light(t, n.light, m);
+    S.surface(t, m, s);
+    const float c0 = c.surf[0] - s[0], c1 = c.surf[1] - s[1], c2 = c.surf[2] - s[2];
+    const float m0 = c.surf[3] - s[3], m1 = c.surf[4] - s[4], m2 = c.surf[5] - s[5], m3 = c.surf[6] - s[6];
+    const float cq = (c0 * c0 + c1 * c1) + c2 * c2, mq = ((m0 * m0 + m1 * m1) + m2 * m2) + m3 * m3;
+    n.step = mq > __uint_as_float(kSameMaterial) ? 0.0f : 1.0f;
+    if (S.skip && t.in && ((n.step == 0.0f && cq == cq) || cq > __uint_as_float(WIDE ? kNearColorWide : kNearColor))) return false;
+    n.color = 1.0f - gclamp(WIDE ? sqrtf(cq) : sqrtf(cq) * 10000.0f, 0.0f, 1.0f);
+    float nn[3], nd;
+    S.normal_depth(t, nn, nd);
+    n.dot = gmax((c.nrm[0] * nn[0] + c.nrm[1] * nn[1]) + c.nrm[2] * nn[2], 0.0f);
+    n.depth = 1.0f - gclamp(fabsf(c.depth - nd) * 4096.0f, 0.0f, 1.0f);
+    far = false;
+    if (S.A.motion) {
+        float mo[2];
+        S.motion(t, mo);
+        const float d0 = c.mo[0] - mo[0], d1 = c.mo[1] - mo[1];
+        far = d0 * d0 + d1 * d1 > __uint_as_float(kSameMotion);
     }
+    return true;
+}
+
+// The attributes of the pixel at (u, v); of a sky pixel (depth 1) only what its
+// output takes, its light and the light's alpha (1 on sky and border texels).
+template <int T>
+VXD void sample_centre(const Sampler<T>& S, float u, float v, Centre& c, float& alpha) {
+    const Tap t = S.tap(u, v);
+    uint32_t m[4];
+    S.light(t, c.light, m);
+    S.normal_depth(t, c.nrm, c.depth);
+    float a[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) a[k] = (m[k] == 0u || m[k] == kBorder) ? 1.0f : 0.0f;
+    alpha = bl(a[0], a[1], a[2], a[3], t.fx, t.fy);
+    if (c.depth == 1.0f) return;
+    S.surface(t, m, c.surf);
+    c.mo[0] = c.mo[1] = 0.0f;
+    if (S.A.motion) S.motion(t, c.mo);
+}
+
+// Loads the tile at S.ox, S.oy with the block's threads; a barrier on both sides.
+template <int T>
+VXD void stage_tile(Sampler<T>& S, Tile<T>& L, uint32_t threads) {
+    constexpr int E = Tile<T>::kEdge;
+    bool odd = false;
+    for (uint32_t k = threadIdx.x; k < (uint32_t)(E * E); k += threads) {
+        const int32_t y = (int32_t)k / E, x = (int32_t)k - y * E;
+        const float4 a = light_at(S.A, S.ox + x, S.oy + y), b = normal_at(S.A, S.ox + x, S.oy + y);
+        L.lm[k] = a;
+        L.nd[k] = b;
+        if (S.A.motion) L.mo[k] = motion_at(S.A, S.ox + x, S.oy + y);
+        const float big = fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(b.x))),
+                                fmaxf(fmaxf(fabsf(b.y), fabsf(b.z)), fabsf(b.w)));
+        const float sum = ((a.x + a.y) + (a.z + b.x)) + ((b.y + b.z) + b.w);   // NaN if any is
+        odd = odd || !(big <= 1.0e15f) || sum != sum;
+    }
+    S.staged = true;
+    S.skip = __syncthreads_or(odd) == 0;
+}
+template <int T>
+VXD void stage_palette(const TaaArgs& A, Tile<T>& L, uint32_t threads) {
+    for (uint32_t k = threadIdx.x; k < (kBorder + 1) * 6; k += threads)
+        L.pal[k] = k >= 6 && k < kBorder * 6 ? A.palette[k] : 0.0f;
+}
+
+// A pixel with history: twelve neighbours on a spiral, the history at (ou, ov)
+// clipped to their range and blended by the running variance.
+template <int T>
+VXD void taa_spiral(const Sampler<T>& S, const Centre& c, size_t i, float u, float v, float ou, float ov, float irx, float iry) {
+    const TaaArgs& A = S.A;
     float last[4];
     sample_last(A, ou, ov, last);
     float lvar = last[3];
-    if (gclamp(ou, 0.0f, 1.0f) != ou || gclamp(ov, 0.0f, 1.0f) != ov) {
-        // out of bounds: this frame's neighbourhood only
-        float count = 0.0f, acc[3] = {0.0f, 0.0f, 0.0f};
-#pragma unroll 1
-        for (int x = -9; x <= 9; ++x) {
-#pragma unroll 1
-            for (int y = -9; y <= 9; ++y) {
-                const float su = gclamp(u + (float)x * irx, 0.001f, 0.999f);
-                const float sv = gclamp(v + (float)y * iry, 0.001f, 0.999f);
-                Sample n;
-                sample_all(A, su, sv, n);
-                float f = gmax((c.nrm[0] * n.nrm[0] + c.nrm[1] * n.nrm[1]) + c.nrm[2] * n.nrm[2], 0.0f);
-                f *= gstep(0.8f, 1.0f - len4(c.matl, n.matl));
-                f *= 1.0f - gclamp(fabsf(c.depth - n.depth) * 4096.0f, 0.0f, 1.0f);
-                f *= 1.0f - gclamp(len3(c.color[0] - n.color[0], c.color[1] - n.color[1], c.color[2] - n.color[2]),
-                                   0.0f, 1.0f);
-                if (len2(c.mo[0] - n.mo[0], c.mo[1] - n.mo[1]) > 0.1f) f = 0.0f;
-                acc[0] = acc[0] + f * n.light[0];
-                acc[1] = acc[1] + f * n.light[1];
-                acc[2] = acc[2] + f * n.light[2];
-                count = count + f;
-            }
-        }
-        o[0] = acc[0] / count; o[1] = acc[1] / count; o[2] = acc[2] / count; o[3] = 1.0f;
-        return;
-    }
+    Near n;
+    bool far;
     float nmin[3] = {10000.0f, 10000.0f, 10000.0f}, nmax[3] = {0.0f, 0.0f, 0.0f}, acc[3] = {0.0f, 0.0f, 0.0f};
     float diff = 1.0f, count = 0.0f;
     const float size = 12.0f;
     float radius = 1.0f;
-    const float noise = rand01(pixkey(A.seed ^ 0x85ebca6bu, A.frame, i), 0u);
+    const float noise = rand01(pixkey(A.seed ^ 0x85ebca6bu, A.frame, (uint32_t)i), 0u);
     const float scale = gclamp(0.1f, 0.5f, 1.0f / c.depth);
 #pragma unroll 1
     for (float angle = (noise * 3.1415f) * 2.118033988749895f; radius <= size; angle = angle + 2.39f) {
@@ -3057,24 +3149,25 @@ __global__ void __launch_bounds__(256) k_light_taa(TaaArgs A) {
         const float rr = radius * (lvar + 1.0f);
         const float su = gclamp(u + ((cs * irx) * rr) * scale, 0.001f, 0.999f);
         const float sv = gclamp(v + ((sn * iry) * rr) * scale, 0.001f, 0.999f);
-        Sample n;
-        sample_all(A, su, sv, n);
-        float f = 1.212f - radius / size;
-        f *= gstep(0.8f, 1.0f - len4(c.matl, n.matl));
-        f *= gmax((c.nrm[0] * n.nrm[0] + c.nrm[1] * n.nrm[1]) + c.nrm[2] * n.nrm[2], 0.0f);
-        f *= 1.0f - gclamp(fabsf(c.depth - n.depth) * 4096.0f, 0.0f, 1.0f);
-        f *= 1.0f - gclamp(len3(c.color[0] - n.color[0], c.color[1] - n.color[1], c.color[2] - n.color[2]) * 10000.0f,
-                           0.0f, 1.0f);
-        if (len2(c.mo[0] - n.mo[0], c.mo[1] - n.mo[1]) > 0.1f) f = 0.0f;
+        const bool same = neighbour<T, false>(S, c, su, sv, n, far);
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
             nmin[k] = gmin(nmin[k], n.light[k]);
             nmax[k] = gmax(nmax[k], n.light[k]);
-            acc[k] = acc[k] + f * n.light[k];
         }
+        if (!same) continue;
+        float f = 1.212f - radius / size;
+        f *= n.step;
+        f *= n.dot;
+        f *= n.depth;
+        f *= n.color;
+        if (far) f = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) acc[k] = acc[k] + f * n.light[k];
         count = count + f;
         diff = diff + len3(n.light[0] - c.light[0], n.light[1] - c.light[1], n.light[2] - c.light[2]) * f;
     }
+    float* o = A.out + 4 * i;
     float cur[3], d[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) cur[k] = (c.light[k] + acc[k]) / (count + 1.0f);
@@ -3093,6 +3186,141 @@ __global__ void __launch_bounds__(256) k_light_taa(TaaArgs A) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) o[k] = cur[k] * (1.0f - t) + last[k] * t;
     o[3] = gclamp(lvar * 0.7f, 0.0f, 1.0f);
+}
+}  // namespace taa
+
+// One block per T x T tile, a wave per 8 x 8 pixels. A pixel takes 13 bilinear
+// samples of 15 attributes around it, at positions of its own: gathered from
+// memory (64-byte records, 16 loads a sample) the L1's one access per cycle
+// bound the pass, 648 us at 1080p with the pass that packed the records. Here
+// the tile's attributes are gathered from LDS, 40 bytes a texel with the palette
+// beside them (colour and material by index), and a sample's normal, depth and
+// motion are read only where its surface is the centre's: 237 us, 16 waves a CU
+// (145 KB of LDS a block) with the vector units busy half of it. A sample past
+// the tile (a variance above 1) reads the G-buffer. Pixels whose history lies
+// off the image are left to k_light_taa_off (A.off: a mask per wave).
+template <int T>
+VXD void light_taa_tile(const TaaArgs& A, taa::Tile<T>& L) {
+    using namespace taa;
+    const uint32_t logical = tile_of_block(A.tiles);
+    if (logical >= A.tiles.ntiles) return;
+    const int32_t x0 = (int32_t)(logical % A.tiles.tiles_x) * T, y0 = (int32_t)(logical / A.tiles.tiles_x) * T;
+    const int32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int32_t wx = x0 + (wave % (T / 8)) * 8, wy = y0 + (wave / (T / 8)) * 8;
+    const int32_t px = wx + (lane & 7), py = wy + (lane >> 3);
+    const bool inside = px < A.width && py < A.height;
+    const size_t i = inside ? (size_t)py * A.width + px : 0;
+    Sampler<T> S{A, L, x0 - Tile<T>::kHalo, y0 - Tile<T>::kHalo, false, false};
+    stage_palette(A, L, T * T);
+    // a tile of sky only passes its light through: no neighbourhood
+    if (__syncthreads_or(inside && A.depth[i] != 1.0f) != 0) stage_tile(S, L, T * T);
+    const float W = (float)A.width, H = (float)A.height;
+    const float u = ((float)px + 0.5f) / W, v = ((float)py + 0.5f) / H;
+    Centre c;
+    float ou = 0.0f, ov = 0.0f;
+    bool surface = false, off = false;
+    if (inside) {
+        float alpha;
+        sample_centre(S, u, v, c, alpha);
+        if (c.depth == 1.0f) {
+            float* o = A.out + 4 * i;
+            o[0] = c.light[0]; o[1] = c.light[1]; o[2] = c.light[2]; o[3] = alpha;
+        } else {
+            surface = true;
+            ou = u + c.mo[0];
+            ov = v + c.mo[1];
+            off = gclamp(ou, 0.0f, 1.0f) != ou || gclamp(ov, 0.0f, 1.0f) != ov;
+        }
+    }
+    const uint64_t offm = __ballot(off);
+    if (lane == 0 && A.motion) A.off[logical * (uint32_t)(T * T / 64) + (uint32_t)wave] = offm;
+    if (surface && !off) taa_spiral<T>(S, c, i, u, v, ou, ov, 1.0f / W, 1.0f / H);
+}
+__global__ void __launch_bounds__(1024) k_light_taa32(TaaArgs A) {
+    __shared__ taa::Tile<32> L;
+    light_taa_tile<32>(A, L);
+}
+__global__ void __launch_bounds__(256) k_light_taa16(TaaArgs A) {
+    __shared__ taa::Tile<16> L;
+    light_taa_tile<16>(A, L);
+}
+
+// Pixels whose history lies off the image take this frame's 19 x 19
+// neighbourhood: 361 samples, their terms added in order. Few pixels are so,
+// near one another: a lane each (in the pass above) made them the end of the
+// launch, 390 of 624 us with 0.15 % of a 1080p image. Here a wave takes one
+// pixel, 64 neighbours together, and four of its lanes then add the terms, one
+// per channel; a block takes up to 16 pixels of an 8 x 8 block (every fourth of
+// those concerned), the blocks of the launch the quarters in turn: 0.2 % of the
+// pixels off the image cost 60 us.
+__global__ void __launch_bounds__(1024) k_light_taa_off(TaaArgs A) {
+    using namespace taa;
+    __shared__ Tile<8> L;
+    __shared__ float terms_s[16][4 * 64];
+    const int32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const float W = (float)A.width, H = (float)A.height;
+    const float irx = 1.0f / W, iry = 1.0f / H;
+    const uint32_t per = (uint32_t)A.tile_waves, n = A.tiles.ntiles * per * 4u;
+    bool palette = false;
+    for (uint32_t k0 = blockIdx.x; k0 < n; k0 += 64u * gridDim.x) {
+        // the block's next 64 quarters, one per lane of every wave
+        const uint32_t mine = k0 + (uint32_t)lane * gridDim.x;
+        const uint64_t mask = mine < n ? A.off[mine >> 2] : 0ull;
+        for (uint64_t some = __ballot(mask != 0ull); some != 0ull; some &= some - 1) {
+            const int32_t from = __builtin_ctzll(some);
+            uint64_t left = (uint64_t)__shfl((unsigned long long)mask, from, 64);
+            const uint32_t item = k0 + (uint32_t)from * gridDim.x, quarter = item & 3u;
+            if (quarter >= (uint32_t)__popcll(left)) continue;
+            const uint32_t k = item >> 2, tile = k / per, w = k - tile * per;
+            const uint32_t edge = per == 16u ? 4u : 2u;   // waves along a tile's edge
+            const int32_t x0 = (int32_t)((tile % A.tiles.tiles_x * edge + w % edge) * 8u);
+            const int32_t y0 = (int32_t)((tile / A.tiles.tiles_x * edge + w / edge) * 8u);
+            if (!palette) stage_palette(A, L, 1024);
+            palette = true;
+            Sampler<8> S{A, L, x0 - Tile<8>::kHalo, y0 - Tile<8>::kHalo, false, false};
+            __syncthreads();
+            stage_tile(S, L, 1024);
+            for (uint32_t turn = 0; left != 0; left &= left - 1, ++turn) {
+                if (turn != (uint32_t)wave * 4u + quarter) continue;
+                const int32_t l = __builtin_ctzll(left);
+                const int32_t px = x0 + (l & 7), py = y0 + (l >> 3);
+                const float u = ((float)px + 0.5f) / W, v = ((float)py + 0.5f) / H;
+                Centre c;
+                float alpha;
+                sample_centre(S, u, v, c, alpha);
+                float acc = 0.0f;   // lane & 3: rgb and the weight
+#pragma unroll 1
+                for (int32_t j0 = 0; j0 < 361; j0 += 64) {
+                    const int32_t j = j0 + lane, x = j / 19 - 9, y = j % 19 - 9;
+                    float* term = terms_s[wave] + 4 * lane;
+                    term[0] = term[1] = term[2] = term[3] = 0.0f;
+                    Near q;
+                    bool far;
+                    if (j < 361 && neighbour<8, true>(S, c, gclamp(u + (float)x * irx, 0.001f, 0.999f),
+                                                      gclamp(v + (float)y * iry, 0.001f, 0.999f), q, far)) {
+                        float f = q.dot;
+                        f *= q.step;
+                        f *= q.depth;
+                        f *= q.color;
+                        if (far) f = 0.0f;
+                        term[0] = f * q.light[0]; term[1] = f * q.light[1]; term[2] = f * q.light[2]; term[3] = f;
+                    }
+                    __builtin_amdgcn_wave_barrier();
+                    const float* terms = terms_s[wave] + (lane & 3);
+#pragma unroll 16
+                    for (int32_t t = 0; t < 64; ++t) acc = acc + terms[4 * t];
+                    __builtin_amdgcn_wave_barrier();
+                }
+                const float count = __shfl(acc, 3, 64);
+                if (lane < 4) A.out[4 * ((size_t)py * A.width + px) + lane] = lane < 3 ? acc / count : 1.0f;
+            }
+        }
+    }
+}
+
+__global__ void __launch_bounds__(256) k_copy_f32(float* dst, const float* src, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256u + threadIdx.x;
+    if (i < n) dst[i] = src[i];
 }
 
 // ===========================================================================
