@@ -251,57 +251,16 @@ struct vx_volume {
     uint64_t* grid;
     int32_t gx, gy, gz;
     size_t ngrid;
+    uint64_t* texels;   // ncells / 8 words (OccView::texels), written with the march grid
 };
-
-// Refreshes the march grid over texel box [t0, t1] (inclusive), clamped to the
-// volume, plus the border cells next to it.
-static hipError_t mgrid_update(const vx_volume* v, const int32_t t0[3], const int32_t t1[3], hipStream_t s) {
-    const int32_t gdim[3] = {v->gx, v->gy, v->gz};
-    const int32_t tdim[3] = {v->sx, v->sy, v->sz};
-    int32_t g0[3], n[3];
-    for (int k = 0; k < 3; ++k) {
-        int32_t lo = std::max(t0[k], 0), hi = std::min(t1[k], tdim[k] - 1);
-        if (hi < lo) return hipSuccess;
-        // fine voxels [2lo, 2hi+1] -> grid cells ((f >> 2) + 1), widened by one cell
-        int32_t c0 = std::max(((2 * lo) >> 2) + 1 - 1, 0);
-        int32_t c1 = std::min(((2 * hi + 1) >> 2) + 1 + 1, gdim[k] - 1);
-        g0[k] = c0;
-        n[k] = c1 - c0 + 1;
-    }
-    size_t total = (size_t)n[0] * n[1] * n[2];
-    OccView V;
-    std::memset(&V, 0, sizeof(V));
-    V.cells = v->cells;
-    V.sx = v->sx; V.sy = v->sy; V.sz = v->sz;
-    V.bx = v->bx; V.by = v->by; V.bz = v->bz;
-    hipLaunchKernelGGL(k_mgrid, dim3((uint32_t)((total + 255) / 256)), dim3(256), 0, s, v->grid, V, v->gx, v->gy,
-                       g0[0], g0[1], g0[2], n[0], n[1], n[2]);
-    return hipGetLastError();
-}
-
-// The whole march grid (every cell, border included).
-static hipError_t mgrid_full(const vx_volume* v, hipStream_t s) {
-    OccView V;
-    std::memset(&V, 0, sizeof(V));
-    V.cells = v->cells;
-    V.sx = v->sx; V.sy = v->sy; V.sz = v->sz;
-    V.bx = v->bx; V.by = v->by; V.bz = v->bz;
-    hipLaunchKernelGGL(k_mgrid, dim3((uint32_t)((v->ngrid + 255) / 256)), dim3(256), 0, s, v->grid, V, v->gx, v->gy,
-                       0, 0, 0, v->gx, v->gy, v->gz);
-    return hipGetLastError();
-}
-
-static inline hipStream_t S(void* s) { return reinterpret_cast<hipStream_t>(s); }
-static inline uint32_t cdiv(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
-
-static vx_status use_device(const vx_ctx* ctx) {
-    VX_HIP(hipSetDevice(ctx->device));
-    return VX_OK;
-}
 
 static OccView occ_view(const vx_volume* v) {
     OccView V;
     V.cells = v->cells;
+    V.texels = v->texels;
+    V.gx = v->gx;
+    V.gxy = v->gx * v->gy;
+    V.grid = v->grid + (size_t)V.gxy + v->gx + 1;
     for (int l = 0; l < 3; ++l) {
         V.lvl[l] = v->lvl[l];
         V.wx[l] = v->wx[l]; V.wy[l] = v->wy[l]; V.wz[l] = v->wz[l];
@@ -310,6 +269,52 @@ static OccView occ_view(const vx_volume* v) {
     V.bx = v->bx; V.by = v->by; V.bz = v->bz;
     V.nlevels = v->nlevels;
     return V;
+}
+
+// Refreshes the march grid and the texel words over the boxes (k_mgrid) that hold
+// grid cells [c0, c1] (inclusive).
+static hipError_t mgrid_cells(const vx_volume* v, const int32_t c0[3], const int32_t c1[3], hipStream_t s) {
+    MgridArgs A;
+    A.grid = v->grid; A.texels = v->texels;
+    A.gx = v->gx; A.gy = v->gy; A.gz = v->gz;
+    for (int k = 0; k < 3; ++k) {
+        const int32_t sh = k == 0 ? 4 : 1;   // grid cell c is cell c - 1, the boxes start at cell -2
+        A.b0[k] = (c0[k] + 1) >> sh;
+        A.n[k] = (uint32_t)(((c1[k] + 1) >> sh) - A.b0[k] + 1);
+    }
+    hipLaunchKernelGGL(k_mgrid, dim3(A.n[1] * A.n[2]), dim3(256), 0, s, A, occ_view(v));
+    return hipGetLastError();
+}
+
+// Refreshes the march grid over texel box [t0, t1] (inclusive), clamped to the
+// volume, plus the border cells next to it.
+static hipError_t mgrid_update(const vx_volume* v, const int32_t t0[3], const int32_t t1[3], hipStream_t s) {
+    const int32_t gdim[3] = {v->gx, v->gy, v->gz};
+    const int32_t tdim[3] = {v->sx, v->sy, v->sz};
+    int32_t c0[3], c1[3];
+    for (int k = 0; k < 3; ++k) {
+        int32_t lo = std::max(t0[k], 0), hi = std::min(t1[k], tdim[k] - 1);
+        if (hi < lo) return hipSuccess;
+        // fine voxels [2lo, 2hi+1] -> grid cells ((f >> 2) + 1), widened by one cell
+        c0[k] = std::max(((2 * lo) >> 2) + 1 - 1, 0);
+        c1[k] = std::min(((2 * hi + 1) >> 2) + 1 + 1, gdim[k] - 1);
+    }
+    return mgrid_cells(v, c0, c1, s);
+}
+
+// The whole march grid (every cell, border included) and every texel word.
+static hipError_t mgrid_full(const vx_volume* v, hipStream_t s) {
+    // (the texel words go one brick further than the grid where 2s + 2 is a multiple of 8)
+    const int32_t c0[3] = {0, 0, 0}, c1[3] = {std::max(v->gx - 1, 2 * v->bx), std::max(v->gy - 1, 2 * v->by), std::max(v->gz - 1, 2 * v->bz)};
+    return mgrid_cells(v, c0, c1, s);
+}
+
+static inline hipStream_t S(void* s) { return reinterpret_cast<hipStream_t>(s); }
+static inline uint32_t cdiv(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
+
+static vx_status use_device(const vx_ctx* ctx) {
+    VX_HIP(hipSetDevice(ctx->device));
+    return VX_OK;
 }
 
 // Length of an XCD's runs of tiles (log2): at most 16 tiles, at least eight runs
@@ -641,6 +646,7 @@ extern "C" vx_status vx_volume_create(vx_ctx* ctx, int32_t sx, int32_t sy, int32
     v->gz = ((2 * sz + 2) >> 2) + 2;
     v->ngrid = (size_t)v->gx * v->gy * v->gz;
     v->grid = nullptr;
+    v->texels = nullptr;
     // The ray-parallel trace addresses the march grid with 32-bit word indices.
     if (v->ngrid >= (size_t(1) << 32)) {
         const size_t words = v->ngrid;
@@ -658,11 +664,13 @@ extern "C" vx_status vx_volume_create(vx_ctx* ctx, int32_t sx, int32_t sy, int32
         if (e == hipSuccess) e = hipMemset(v->lvl[l], 0, nw * 8);
     }
     if (e == hipSuccess) e = dev_malloc(&v->grid, v->ngrid * 8);
+    if (e == hipSuccess) e = dev_malloc(&v->texels, v->ncells);
     if (e == hipSuccess) e = mgrid_full(v, nullptr);
     if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         (void)hipFree(v->cells);
         (void)hipFree(v->grid);
+        (void)hipFree(v->texels);
         for (int l = 0; l < 3; ++l) (void)hipFree(v->lvl[l]);
         delete v;
         return fail(VX_ERR_OUT_OF_MEMORY, "volume allocation failed: %s", hipGetErrorString(e));
@@ -676,6 +684,7 @@ extern "C" vx_status vx_volume_destroy(vx_volume* v) {
     (void)hipSetDevice(v->ctx->device);
     (void)hipFree(v->cells);
     (void)hipFree(v->grid);
+    (void)hipFree(v->texels);
     for (int l = 0; l < 3; ++l) (void)hipFree(v->lvl[l]);
     delete v;
     return VX_OK;
@@ -693,11 +702,11 @@ extern "C" vx_status vx_volume_clear(vx_volume* v, void* stream) {
     if (vx_status st = use_device(v->ctx)) return st;
     ClearArgs A;
     std::memset(&A, 0, sizeof(A));
-    uint64_t* p[4] = {v->cells, v->lvl[0], v->lvl[1], v->lvl[2]};
+    uint64_t* p[5] = {v->cells, v->texels, v->lvl[0], v->lvl[1], v->lvl[2]};
     uint64_t blocks = 0;
-    for (int k = 0; k <= v->nlevels; ++k) {
+    for (int k = 0; k < 2 + v->nlevels; ++k) {
         A.p[k] = p[k];
-        A.words[k] = k == 0 ? v->ncells : (size_t)v->wx[k - 1] * v->wy[k - 1] * v->wz[k - 1];
+        A.words[k] = k == 0 ? v->ncells : (k == 1 ? v->ncells / 8 : (size_t)v->wx[k - 2] * v->wy[k - 2] * v->wz[k - 2]);
         A.blocks[k] = cdiv(A.words[k], 512);
         blocks += A.blocks[k];
     }

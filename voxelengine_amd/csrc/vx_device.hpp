@@ -167,6 +167,13 @@ VXD void tangent_frame(f3 n, f3& t, f3& b) {
 // ---------------------------------------------------------------------------
 struct OccView {
     const uint64_t* cells;
+    // A word per brick (cells' order), a bit per texel of it that holds a voxel:
+    // texel (x, y, z) of the brick at bit 63 - (x | y << 2 | z << 4), so that a
+    // left shift moves it to the sign bit. Texels outside [0, s) are 0.
+    const uint64_t* texels;
+    // The march grid at voxel (0, 0, 0) (k_mgrid), its pitches in words.
+    const uint64_t* grid;
+    int32_t gx, gxy;
     const uint64_t* lvl[3];
     int32_t sx, sy, sz;        // texel dims
     int32_t bx, by, bz;        // brick grid (padded)

@@ -26,14 +26,23 @@ struct LevelRanges {
     uint16_t r[kLevelRanges][6];
 };
 
-// The arrays of a volume (cells, levels 1..3, march grid) to be emptied.
+// The arrays of a volume (cells, texels, levels 1..3, march grid) to be emptied.
 struct ClearArgs {
-    uint64_t* p[4];
-    size_t words[4];
-    uint32_t blocks[4];                // 512 words each
+    uint64_t* p[5];
+    size_t words[5];
+    uint32_t blocks[5];                // 512 words each
     uint64_t* grid;
     size_t ngrid;
     int32_t gx, gy;
+};
+
+// Boxes of 16 x 2 x 2 cells whose march grid words and texel words are rewritten.
+struct MgridArgs {
+    uint64_t* grid;
+    uint64_t* texels;
+    int32_t gx, gy, gz;
+    int32_t b0[3];
+    uint32_t n[3];
 };
 
 // Block -> pixel tile mapping (16x16 pixels per 256-thread block; tile_of_block).
@@ -306,8 +315,7 @@ __global__ void __launch_bounds__(256) k_shade_bwd_batch(const ShadeArgs* items,
 __global__ void k_shade_bwd_finish(const long long* acc, float* dpal, float* dlight);
 __global__ void k_zero_i64(long long* p, int n);
 
-__global__ void __launch_bounds__(256) k_mgrid(uint64_t* grid, OccView V, int32_t gx, int32_t gy, int32_t g0x, int32_t g0y,
-                                               int32_t g0z, int32_t nx, int32_t ny, int32_t nz);
+__global__ void __launch_bounds__(256) k_mgrid(MgridArgs A, OccView V);
 
 // Ray-parallel trace, instantiated for 256/512-thread blocks and 2/4/8 DDA
 // steps between refills; launch_march enqueues march, listed rays and resolve
