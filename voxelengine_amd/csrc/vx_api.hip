@@ -409,6 +409,8 @@ extern "C" vx_status vx_ctx_create(int32_t device, vx_ctx** out) {
     c->rb_ops = nullptr;
     c->rb_ops_cap = 0;
     hipError_t me = dev_malloc(&c->grad_acc, (256 * 6 + 6) * sizeof(long long));
+    // (the adjoint's accumulator: 0 before a call, cleared by its last kernel)
+    if (me == hipSuccess) me = hipMemset(c->grad_acc, 0, (256 * 6 + 6) * sizeof(long long));
     if (me == hipSuccess) me = dev_malloc(&c->march.counters, kCounterWords * sizeof(uint32_t));
     if (me != hipSuccess) {
         (void)hipFree(c->grad_acc);
@@ -1891,6 +1893,9 @@ extern "C" vx_status vx_shade_forward(vx_ctx* ctx, const vx_view* view, const vx
     return VX_OK;
 }
 
+// Blocks of the adjoint of a view: one per CU at most (k_shade_bwd).
+static uint32_t shade_blocks(uint32_t npx) { return std::min<uint32_t>(cdiv(npx, 1024), 256); }
+
 extern "C" vx_status vx_shade_backward(vx_ctx* ctx, const vx_view* view, const vx_gbuf* g, const vx_trace_out* vis,
                                        const float* ssao, const float* palette, const float light[6],
                                        const float* dl_drgb, float* dpalette, float* dlight, void* stream) {
@@ -1900,9 +1905,7 @@ extern "C" vx_status vx_shade_backward(vx_ctx* ctx, const vx_view* view, const v
     if (vx_status st = use_device(ctx)) return st;
     A.dl_drgb = dl_drgb;
     const int nacc = 256 * 6 + 6;
-    hipLaunchKernelGGL(k_zero_i64, dim3(cdiv(nacc, 256)), dim3(256), 0, S(stream), ctx->grad_acc, nacc);
-    uint32_t grid = std::min<uint32_t>(cdiv(A.npx, 256), 1024);
-    hipLaunchKernelGGL(k_shade_bwd, dim3(grid), dim3(256), 0, S(stream), A, ctx->grad_acc);
+    hipLaunchKernelGGL(k_shade_bwd, dim3(shade_blocks(A.npx)), dim3(1024), 0, S(stream), A, ctx->grad_acc);
     hipLaunchKernelGGL(k_shade_bwd_finish, dim3(cdiv(nacc, 256)), dim3(256), 0, S(stream), ctx->grad_acc, dpalette,
                        dlight);
     VX_LAUNCHED("k_shade_bwd");
@@ -1923,7 +1926,7 @@ static vx_status vx_shade_backward_batch_impl(vx_ctx* ctx, const vx_shade_item* 
         if (vx_status st = shade_args(&it.view, &it.gbuf, &it.vis, it.ssao, palette, light, h[i])) return st;
         h[i].dl_drgb = it.dl_drgb;
         b0[i] = (uint32_t)blocks;
-        blocks += std::min<uint32_t>(cdiv(h[i].npx, 256), 1024);
+        blocks += shade_blocks(h[i].npx);
     }
     b0[n] = (uint32_t)blocks;
     if (vx_status st = use_device(ctx)) return st;
@@ -1943,8 +1946,7 @@ static vx_status vx_shade_backward_batch_impl(vx_ctx* ctx, const vx_shade_item* 
     VX_HIP(hipMemcpyAsync(ctx->shade_block0, b0.data(), (n + 1) * sizeof(uint32_t), hipMemcpyHostToDevice,
                           S(stream)));
     const int nacc = 256 * 6 + 6;
-    hipLaunchKernelGGL(k_zero_i64, dim3(cdiv(nacc, 256)), dim3(256), 0, S(stream), ctx->grad_acc, nacc);
-    hipLaunchKernelGGL(k_shade_bwd_batch, dim3((uint32_t)blocks), dim3(256), 0, S(stream), ctx->shade_items,
+    hipLaunchKernelGGL(k_shade_bwd_batch, dim3((uint32_t)blocks), dim3(1024), 0, S(stream), ctx->shade_items,
                        ctx->shade_block0, n, ctx->grad_acc);
     hipLaunchKernelGGL(k_shade_bwd_finish, dim3(cdiv(nacc, 256)), dim3(256), 0, S(stream), ctx->grad_acc, dpalette,
                        dlight);

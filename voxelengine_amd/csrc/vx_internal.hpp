@@ -309,11 +309,10 @@ __global__ void __launch_bounds__(256) k_light_taa16(TaaArgs A);
 __global__ void __launch_bounds__(1024) k_light_taa_off(TaaArgs A);
 __global__ void __launch_bounds__(256) k_copy_f32(float* dst, const float* src, size_t n);
 __global__ void k_shade_fwd(ShadeArgs A);
-__global__ void __launch_bounds__(256) k_shade_bwd(ShadeArgs A, long long* acc);
-__global__ void __launch_bounds__(256) k_shade_bwd_batch(const ShadeArgs* items, const uint32_t* block0, uint32_t n,
-                                                         long long* acc);
-__global__ void k_shade_bwd_finish(const long long* acc, float* dpal, float* dlight);
-__global__ void k_zero_i64(long long* p, int n);
+__global__ void __launch_bounds__(1024) k_shade_bwd(ShadeArgs A, long long* acc);
+__global__ void __launch_bounds__(1024) k_shade_bwd_batch(const ShadeArgs* items, const uint32_t* block0, uint32_t n,
+                                                          long long* acc);
+__global__ void k_shade_bwd_finish(long long* acc, float* dpal, float* dlight);
 
 __global__ void __launch_bounds__(256) k_mgrid(MgridArgs A, OccView V);
 
