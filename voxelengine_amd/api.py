@@ -125,6 +125,14 @@ def region_tuple(r: L.Region):
     return (r.x, r.y, r.z, r.w, r.h, r.d)
 
 
+def _regions(regions):
+    """ctypes array of (x, y, z, w, h, d) regions."""
+    if all(len(r) == 6 for r in regions):
+        a = np.array([tuple(r) for r in regions], np.int64).astype(np.int32)
+        return (L.Region * len(regions)).from_buffer(a)
+    return (L.Region * len(regions))(*[L.Region(*r) for r in regions])
+
+
 def make_instance(model_ptr: int, dims, prev, cur, pivot=(0.0, 0.0, 0.0), flags=L.INST_UPDATE) -> L.Instance:
     inst = L.Instance()
     inst.model = model_ptr
@@ -137,6 +145,9 @@ def make_instance(model_ptr: int, dims, prev, cur, pivot=(0.0, 0.0, 0.0), flags=
 
 
 IDENTITY = np.eye(4, dtype=np.float32).reshape(16)
+
+
+REGION_DTYPE = np.dtype([("x", "<i4"), ("y", "<i4"), ("z", "<i4"), ("w", "<u4"), ("h", "<u4"), ("d", "<u4")])
 
 
 class Volume:
@@ -169,11 +180,11 @@ class Volume:
         dirty = (L.Region * max(n, 1))()
         nd = C.c_uint32()
         check(L.lib().vx_volume_rebuild(self.h, arr, n, threshold, dirty, C.byref(nd), _stream(stream)))
-        return [region_tuple(dirty[i]) for i in range(nd.value)]
+        return np.frombuffer(dirty, REGION_DTYPE)[:nd.value].tolist()   # (x, y, z, w, h, d) tuples
 
     def build_levels(self, regions=None, stream=None):
         if regions:
-            arr = (L.Region * len(regions))(*[L.Region(*r) for r in regions])
+            arr = _regions(regions)
             check(L.lib().vx_volume_build_levels(self.h, arr, len(regions), _stream(stream)))
         else:
             check(L.lib().vx_volume_build_levels(self.h, None, 0, _stream(stream)))
@@ -197,14 +208,17 @@ class Volume:
         return out
 
 
+_MATRICES = ("last_view", "view", "inv_view", "proj", "inv_proj")
+
+
 def view_struct(vd: dict) -> L.View:
-    v = L.View()
-    for k in ("last_view", "view", "inv_view", "proj", "inv_proj"):
-        setattr(v, k, L.f16(*np.asarray(vd[k], np.float32).reshape(16)))
-    v.res = (C.c_float * 2)(*[float(x) for x in vd["res"]])
-    v.ires = (C.c_float * 2)(*[float(x) for x in vd["ires"]])
-    v.cam_pos = (C.c_float * 3)(*[float(x) for x in vd["cam_pos"]])
-    v.jitter = (C.c_float * 2)(*[float(x) for x in vd["jitter"]])
+    # as bytes: 80 matrix elements as ctypes values took 11 us, half a small call
+    mats = [vd[k] for k in _MATRICES]
+    if not all(type(m) is np.ndarray and m.dtype == np.float32 and m.size == 16 for m in mats):
+        mats = [np.asarray(m, np.float32).reshape(16) for m in mats]
+    (rx, ry), (ix, iy), (x, y, z), (jx, jy) = vd["res"], vd["ires"], vd["cam_pos"], vd["jitter"]
+    rest = np.array((rx, ry, ix, iy, x, y, z, jx, jy), np.float32)
+    v = L.View.from_buffer_copy(b"".join([m.tobytes() for m in mats]) + rest.tobytes() + bytes(12))
     v.frame, v.width, v.height = vd["frame"], vd["width"], vd["height"]
     return v
 
