@@ -1114,7 +1114,7 @@ extern "C" vx_status vx_primary(vx_ctx* ctx, const vx_model* model, const vx_vie
     mat_mul_f32(view->proj, view->view, A.pv);
     for (int k = 0; k < 3; ++k) { A.mips[k] = model->mip[k]; A.dims[k] = model->dims[k]; }
     A.pos = g->pos; A.nrm = g->normal; A.mat = g->material;
-    hipLaunchKernelGGL(k_primary, dim3(A.tiles.blocks), dim3(256), 0, S(stream), A);
+    launch_primary(S(stream), A);
     VX_LAUNCHED("k_primary");
     return VX_OK;
 }

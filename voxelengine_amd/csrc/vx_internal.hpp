@@ -298,7 +298,7 @@ __global__ void __launch_bounds__(256) k_light_count(LightArgs A, LightListArgs 
 __global__ void __launch_bounds__(256) k_light_records(LightArgs A, LightListArgs B);
 __global__ void __launch_bounds__(256) k_light_march(OccView V, LightArgs A, LightListArgs B);
 __global__ void __launch_bounds__(256) k_light_fold(LightArgs A, LightListArgs B);
-__global__ void __launch_bounds__(256) k_primary(PrimaryArgs A);
+void launch_primary(hipStream_t s, const PrimaryArgs& A);
 __global__ void __launch_bounds__(256) k_reflection(OccView V, ReflectionArgs A);
 __global__ void __launch_bounds__(256) k_gbuf_depth(DepthArgs A);
 __global__ void __launch_bounds__(256) k_ssao(SsaoArgs A);

@@ -2633,9 +2633,22 @@ struct MipRay {
     int32_t left[3];
     uint32_t idx;
 };
-// One step along the axes whose t_max is the least (each lane its own).
+// One step along the axes whose t_max is the least (each lane its own). FEW: as
+// selects, more vector instructions but no scalar ones between them.
+template <bool FEW>
 VXD void mip_step(MipRay& R, const float td[3], const int32_t stride[3]) {
     const float t = fminf(fminf(R.t[0], R.t[1]), R.t[2]);
+    if (FEW) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const bool m = R.t[k] == t;
+            const float nt = R.t[k] + td[k];
+            R.t[k] = m ? nt : R.t[k];
+            R.left[k] -= m ? 1 : 0;
+            R.idx += (uint32_t)(m ? stride[k] : 0);
+        }
+        return;
+    }
     const uint64_t m0 = __ballot(R.t[0] == t), m1 = __ballot(R.t[1] == t), m2 = __ballot(R.t[2] == t);
     uint64_t sv;
     asm volatile(
@@ -2659,7 +2672,7 @@ VXD void mip_step(MipRay& R, const float td[3], const int32_t stride[3]) {
           [s0] "v"(stride[0]), [s1] "v"(stride[1]), [s2] "v"(stride[2]));
 }
 
-template <int K>
+template <int K, bool FEW>
 VXD int32_t intersect_volume_fast(const ModelMips& A, const float res[2], int32_t frame, f3 o3, f3 d3, f3 cam,
                                   float uvx, float uvy, f3& hit, f3& nrm, uint32_t& material) {
     float o[3] = {o3.x, o3.y, o3.z};
@@ -2716,7 +2729,7 @@ VXD int32_t intersect_volume_fast(const ModelMips& A, const float res[2], int32_
             bool out[K];
 #pragma unroll
             for (int u = 0; u < K; ++u) {
-                mip_step(R, td, stride);
+                mip_step<FEW>(R, td, stride);
                 out[u] = (R.left[0] | R.left[1] | R.left[2]) < 0;
                 vb[u] = base[min(R.idx, last)];
             }
@@ -2737,7 +2750,7 @@ VXD int32_t intersect_volume_fast(const ModelMips& A, const float res[2], int32_
             // step e of the group again
             R = R0;
 #pragma unroll 1
-            for (int u = 0; u < e; ++u) mip_step(R, td, stride);
+            for (int u = 0; u < e; ++u) mip_step<FEW>(R, td, stride);
             const float t = fminf(fminf(R.t[0], R.t[1]), R.t[2]);
             float sel[3];
 #pragma unroll
@@ -2767,7 +2780,7 @@ VXD int32_t intersect_volume_fast(const ModelMips& A, const float res[2], int32_
                 return 1;
             }
             // a glass voxel the dither lets through: the march goes on after it
-            mip_step(R, td, stride);
+            mip_step<FEW>(R, td, stride);
             n += e + 1;
             if (n >= 512) return 0;
         }
@@ -2780,13 +2793,18 @@ VXD int32_t intersect_volume_fast(const ModelMips& A, const float res[2], int32_
 // band per XCD; 541 with this one, 420 with tiles dealt over the XCDs (4, 12 and
 // 16 steps per group: 4, 1 and 5 % slower). 68 draws at 1080p, k_primary_inst:
 // 393, 311 and 182 us (8 steps: 3 % slower, small models end within four).
-constexpr int kPrimarySteps = 8, kInstanceSteps = 4;
+//
+// A launch whose waves are all resident at once lasts as long as its longest
+// ray's chain of steps: 16 steps per group, as selects. 512^3, 640x360: 208 us
+// with 8 steps and exec, 191 with 16, 175 as selects too; 960x540: 230, 219, 208;
+// 1280x720: 280, 270, 265 but at 256^3 149, 153, 163; 1920x1080: 418, 419, 435.
+constexpr int kPrimarySteps = 8, kPrimaryFewSteps = 16, kInstanceSteps = 4;
 
-template <int K>
+template <int K, bool FEW>
 VXD int32_t intersect_volume(const ModelMips& A, const float res[2], int32_t frame, f3 o3, f3 d3, f3 cam,
                              float uvx, float uvy, f3& hit, f3& nrm, uint32_t& material) {
     if ((uint64_t)(uint32_t)A.dims[0] * (uint32_t)A.dims[1] * (uint32_t)A.dims[2] < (1ull << 32) && primary_fast_ok(o3, d3))
-        return intersect_volume_fast<K>(A, res, frame, o3, d3, cam, uvx, uvy, hit, nrm, material);
+        return intersect_volume_fast<K, FEW>(A, res, frame, o3, d3, cam, uvx, uvy, hit, nrm, material);
     return intersect_volume_any(A, res, frame, o3, d3, cam, uvx, uvy, hit, nrm, material);
 }
 
@@ -2853,6 +2871,7 @@ VXD bool box_far_face_drawn(const int32_t dims[3], f3 lc, f3 dl, const float* wo
     return ce[3] >= 0.1f;
 }
 
+template <bool FEW>
 __global__ void __launch_bounds__(256) k_primary(PrimaryArgs A) {
     int32_t px, py;
     if (!tile_pixel(A.tiles, px, py)) return;
@@ -2871,7 +2890,7 @@ __global__ void __launch_bounds__(256) k_primary(PrimaryArgs A) {
     // the camera) stays empty
     if (box_far_face_drawn(M.dims, cam, dir, nullptr, A.pv)) {
         f3 start = clip_to_aabb(cam, dir, M.dims);
-        h = intersect_volume<kPrimarySteps>(M, vw.res, vw.frame, start, dir, cam, ndc_x, ndc_y, hit, nrm, mat);
+        h = intersect_volume<FEW ? kPrimaryFewSteps : kPrimarySteps, FEW>(M, vw.res, vw.frame, start, dir, cam, ndc_x, ndc_y, hit, nrm, mat);
     }
     if (!h) {
         hit = mk3(0.0f, 0.0f, 0.0f);
@@ -2881,6 +2900,12 @@ __global__ void __launch_bounds__(256) k_primary(PrimaryArgs A) {
     A.pos[3 * i + 0] = hit.x; A.pos[3 * i + 1] = hit.y; A.pos[3 * i + 2] = hit.z;
     A.nrm[3 * i + 0] = nrm.x; A.nrm[3 * i + 1] = nrm.y; A.nrm[3 * i + 2] = nrm.z;
     A.mat[i] = (uint8_t)mat;
+}
+
+// (2048 blocks: eight waves a SIMD)
+void launch_primary(hipStream_t s, const PrimaryArgs& A) {
+    if (A.tiles.blocks <= 2048u) hipLaunchKernelGGL(k_primary<true>, dim3(A.tiles.blocks), dim3(256), 0, s, A);
+    else hipLaunchKernelGGL(k_primary<false>, dim3(A.tiles.blocks), dim3(256), 0, s, A);
 }
 
 // ===========================================================================
@@ -2958,7 +2983,7 @@ __global__ void __launch_bounds__(256) k_primary_inst(PrimaryInstArgs A) {
         const f3 start = clip_to_aabb(lc, dl, I.m.dims);
         f3 hit, nrm;
         uint32_t mat = 0;
-        if (!intersect_volume<kInstanceSteps>(I.m, vw.res, vw.frame, start, dl, lc, ndc_x, ndc_y, hit, nrm, mat)) continue;
+        if (!intersect_volume<kInstanceSteps, false>(I.m, vw.res, vw.frame, start, dl, lc, ndc_x, ndc_y, hit, nrm, mat)) continue;
         float h4[4] = {hit.x * 0.1f, hit.y * 0.1f, hit.z * 0.1f, 1.0f}, wh[4], cur[4];
         mat_vec(I.w, h4, wh);
         mat_vec(A.pv, wh, cur);
