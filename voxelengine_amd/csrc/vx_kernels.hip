@@ -3151,24 +3151,26 @@ struct Sampler {
         mo[0] = bl(q[0].x, q[1].x, q[2].x, q[3].x, t.fx, t.fy);
         mo[1] = bl(q[0].y, q[1].y, q[2].y, q[3].y, t.fx, t.fy);
     }
-    // Colour and material (its fourth channel is 1 on the border, 0 inside).
+    // Channels FROM .. TO - 1 of colour (0..2) and material (3..6, the last 1 on
+    // the border and 0 inside).
+    template <int FROM, int TO>
     VXD void surface(const Tap& t, const uint32_t m[4], float s[7]) const {
         if (m[0] == m[1] && m[0] == m[2] && m[0] == m[3]) {   // bl of one value, its two halves equal
             const float* e = L.pal + 6 * m[0];
 #pragma unroll
-            for (int c = 0; c < 7; ++c) {
+            for (int c = FROM; c < TO; ++c) {
                 const float a = c < 6 ? e[c] : (m[0] == kBorder ? 1.0f : 0.0f);
                 const float r = a * (1.0f - t.fx) + a * t.fx;
                 s[c] = r * (1.0f - t.fy) + r * t.fy;
             }
         } else {
 #pragma unroll
-            for (int c = 0; c < 6; ++c)
-                s[c] = bl(L.pal[6 * m[0] + c], L.pal[6 * m[1] + c], L.pal[6 * m[2] + c], L.pal[6 * m[3] + c], t.fx, t.fy);
-            float b[4];
+            for (int c = FROM; c < TO; ++c) {
+                float q[4];
 #pragma unroll
-            for (int k = 0; k < 4; ++k) b[k] = m[k] == kBorder ? 1.0f : 0.0f;
-            s[6] = bl(b[0], b[1], b[2], b[3], t.fx, t.fy);
+                for (int k = 0; k < 4; ++k) q[k] = c < 6 ? L.pal[6 * m[k] + c] : (m[k] == kBorder ? 1.0f : 0.0f);
+                s[c] = bl(q[0], q[1], q[2], q[3], t.fx, t.fy);
+            }
         }
     }
 };
@@ -3220,12 +3222,16 @@ VXD bool neighbour(const Sampler<T>& S, const Centre& c, float u, float v, Near&
     uint32_t m[4];
     float s[7];
     S.light(t, n.light, m);
-    S.surface(t, m, s);
+    const bool skip = S.skip && t.in;
+    S.template surface<0, 3>(t, m, s);
     const float c0 = c.surf[0] - s[0], c1 = c.surf[1] - s[1], c2 = c.surf[2] - s[2];
+    const float cq = (c0 * c0 + c1 * c1) + c2 * c2;
+    if (skip && cq > __uint_as_float(WIDE ? kNearColorWide : kNearColor)) return false;
+    S.template surface<3, 7>(t, m, s);
     const float m0 = c.surf[3] - s[3], m1 = c.surf[4] - s[4], m2 = c.surf[5] - s[5], m3 = c.surf[6] - s[6];
-    const float cq = (c0 * c0 + c1 * c1) + c2 * c2, mq = ((m0 * m0 + m1 * m1) + m2 * m2) + m3 * m3;
+    const float mq = ((m0 * m0 + m1 * m1) + m2 * m2) + m3 * m3;
     n.step = mq > __uint_as_float(kSameMaterial) ? 0.0f : 1.0f;
-    if (S.skip && t.in && ((n.step == 0.0f && cq == cq) || cq > __uint_as_float(WIDE ? kNearColorWide : kNearColor))) return false;
+    if (skip && n.step == 0.0f && cq == cq) return false;
     n.color = 1.0f - gclamp(WIDE ? sqrtf(cq) : sqrtf(cq) * 10000.0f, 0.0f, 1.0f);
     float nn[3], nd;
     S.normal_depth(t, nn, nd);
@@ -3254,7 +3260,7 @@ VXD void sample_centre(const Sampler<T>& S, float u, float v, Centre& c, float& 
     for (int k = 0; k < 4; ++k) a[k] = (m[k] == 0u || m[k] == kBorder) ? 1.0f : 0.0f;
     alpha = bl(a[0], a[1], a[2], a[3], t.fx, t.fy);
     if (c.depth == 1.0f) return;
-    S.surface(t, m, c.surf);
+    S.template surface<0, 7>(t, m, c.surf);
     c.mo[0] = c.mo[1] = 0.0f;
     if (S.A.motion) S.motion(t, c.mo);
 }
@@ -3264,16 +3270,32 @@ template <int T>
 VXD void stage_tile(Sampler<T>& S, Tile<T>& L, uint32_t threads) {
     constexpr int E = Tile<T>::kEdge;
     bool odd = false;
-    for (uint32_t k = threadIdx.x; k < (uint32_t)(E * E); k += threads) {
-        const int32_t y = (int32_t)k / E, x = (int32_t)k - y * E;
-        const float4 a = light_at(S.A, S.ox + x, S.oy + y), b = normal_at(S.A, S.ox + x, S.oy + y);
-        L.lm[k] = a;
-        L.nd[k] = b;
-        if (S.A.motion) L.mo[k] = motion_at(S.A, S.ox + x, S.oy + y);
-        const float big = fmaxf(fmaxf(fmaxf(fabsf(a.x), fabsf(a.y)), fmaxf(fabsf(a.z), fabsf(b.x))),
-                                fmaxf(fmaxf(fabsf(b.y), fabsf(b.z)), fabsf(b.w)));
-        const float sum = ((a.x + a.y) + (a.z + b.x)) + ((b.y + b.z) + b.w);   // NaN if any is
-        odd = odd || !(big <= 1.0e15f) || sum != sum;
+    // four texels of a thread are in flight together: one latency for a tile of 32
+    for (uint32_t k0 = threadIdx.x; k0 < (uint32_t)(E * E); k0 += 4u * threads) {
+        float4 a[4], b[4];
+        float2 mo[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            // (a texel past the tile reads its last one and is dropped)
+            const uint32_t k = min(k0 + j * threads, (uint32_t)(E * E - 1));
+            const int32_t y = (int32_t)k / E, x = (int32_t)k - y * E;
+            a[j] = light_at(S.A, S.ox + x, S.oy + y);
+            b[j] = normal_at(S.A, S.ox + x, S.oy + y);
+            mo[j] = motion_at(S.A, S.ox + x, S.oy + y);
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t k = k0 + j * threads;
+            if (k < (uint32_t)(E * E)) {
+                L.lm[k] = a[j];
+                L.nd[k] = b[j];
+                L.mo[k] = mo[j];
+            }
+            const float big = fmaxf(fmaxf(fmaxf(fabsf(a[j].x), fabsf(a[j].y)), fmaxf(fabsf(a[j].z), fabsf(b[j].x))),
+                                    fmaxf(fmaxf(fabsf(b[j].y), fabsf(b[j].z)), fabsf(b[j].w)));
+            const float sum = ((a[j].x + a[j].y) + (a[j].z + b[j].x)) + ((b[j].y + b[j].z) + b[j].w);   // NaN if any is
+            odd = odd || !(big <= 1.0e15f) || sum != sum;
+        }
     }
     S.staged = true;
     S.skip = __syncthreads_or(odd) == 0;
@@ -3354,8 +3376,8 @@ VXD void taa_spiral(const Sampler<T>& S, const Centre& c, size_t i, float u, flo
 // bound the pass, 648 us at 1080p with the pass that packed the records. Here
 // the tile's attributes are gathered from LDS, 40 bytes a texel with the palette
 // beside them (colour and material by index), and a sample's normal, depth and
-// motion are read only where its surface is the centre's: 237 us, 16 waves a CU
-// (145 KB of LDS a block) with the vector units busy half of it. A sample past
+// motion are read only where its colour and material are the centre's: 207 us, 16
+// waves a CU (145 KB of LDS a block) with the vector units busy half of it. A sample past
 // the tile (a variance above 1) reads the G-buffer. Pixels whose history lies
 // off the image are left to k_light_taa_off (A.off: a mask per wave).
 template <int T>
