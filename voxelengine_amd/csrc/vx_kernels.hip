@@ -1768,7 +1768,7 @@ __global__ void __launch_bounds__(256) k_resolve(MarchArgs A) {
 // fetches only where a ray enters another cell): trace_tile_waves draws the
 // line. Whole vx_trace calls before and after: 61x43 pixels of 64^3, 6 DDA
 // rays each, 124 -> 24 us; 320x180 of 512^3, 6 rays, 142 -> 41 us; 61x43 of
-// 512^3, 1 Sparse + 16 SuperSparse + 1, 275 -> 55 us (one thread per pixel).
+// 512^3, 1 Sparse + 16 SuperSparse + 1, 275 (one thread per pixel) -> 22 us.
 // ===========================================================================
 constexpr int kTileAhead = 4;      // voxels (DDA) per fetch latency
 constexpr int kTileSparse = 8;     // positions of a sparse march per fetch latency
@@ -1938,9 +1938,9 @@ __global__ void __launch_bounds__(64 * kTileMaxWaves) k_trace_tile(MarchArgs A) 
 // at most two chips of waves (256 CUs x 32 waves); whole calls, tile against
 // ring: 16200 waves 136 / 162 us, 18000 waves 100 / 113 us (4 AO rays to 16) but
 // 43200 waves 307 / 207 us and 64800 waves 357 / 218 us. Sparse marchers: as
-// many waves as fill the chip once (more of them repeat a pixel's set-up: 640x360
-// with 1 + 4 rays 63 us at 2 waves per tile, 68 at 4, 75 at 5), and the
-// per-pixel kernel once one wave per tile does.
+// many waves as fill the chip once (more of them repeat a pixel's set-up), and
+// the per-pixel kernel once one wave per tile does: 640x360 with 1 + 4 rays 37 us
+// at 2 waves per tile, 41 per pixel; 960x540 118 at 4 waves, 64 per pixel.
 uint32_t trace_tile_waves(uint32_t ntiles, int32_t nrays, bool all_dda) {
     constexpr uint32_t kChipWaves = 8192;
     if (nrays == 0) return 1;
