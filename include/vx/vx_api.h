@@ -414,7 +414,9 @@ typedef struct {
  * same-surface neighbours, the last frame's light (at uv + motion) clipped to
  * the neighbourhood's range and blended by the running variance; pixels whose
  * last position left the screen average a 19x19 same-surface neighbourhood.
- * Uses view width/height and frame; seed keys the per-pixel spiral angle. */
+ * Uses view width/height and frame; seed keys the per-pixel spiral angle. An out
+ * that overlaps an input other than last is written through scratch (16 bytes
+ * per pixel, allocated by the first such call). */
 vx_status vx_light_taa(vx_ctx* ctx, const vx_view* view, const vx_taa_io* io, uint32_t seed, void* stream);
 
 /* ---------------------------------------------------------------- reflection pass

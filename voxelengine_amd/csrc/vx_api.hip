@@ -203,7 +203,7 @@ struct vx_ctx {
     float* taa_out;          // LightTAA: the output of a pass that overwrites one of its inputs
     uint32_t taa_cap;
     uint64_t* taa_off;       // LightTAA: masks of the pixels whose history lies off the image
-    uint32_t taa_off_cap;
+    uint32_t taa_off_px;     // enough of them for images of this many pixels
     // light pass ray list: per pixel first record and count, the total, the records
     uint32_t* lt_first;
     uint32_t* lt_count;
@@ -395,7 +395,7 @@ extern "C" vx_status vx_ctx_create(int32_t device, vx_ctx** out) {
     c->taa_out = nullptr;
     c->taa_cap = 0;
     c->taa_off = nullptr;
-    c->taa_off_cap = 0;
+    c->taa_off_px = 0;
     c->lt_first = c->lt_count = c->lt_total = nullptr;
     c->lt_px_cap = 0;
     c->lt_rec = nullptr;
@@ -1345,13 +1345,15 @@ extern "C" vx_status vx_light_taa(vx_ctx* ctx, const vx_view* view, const vx_taa
         A.tile_waves = 16;
     }
     const uint32_t masks = A.tiles.ntiles * (uint32_t)A.tile_waves;
-    if (io->motion && ctx->taa_off_cap < masks) {
+    if (ctx->taa_off_px < npx) {
+        // masks of any image of npx pixels: (w / 32 + 1) (h / 32 + 1) 16 at most
+        const size_t most = npx / 64u + (16386u + npx / 16384u) / 2u + 64u;
         VX_HIP(hipDeviceSynchronize());
         (void)hipFree(ctx->taa_off);
         ctx->taa_off = nullptr;
-        ctx->taa_off_cap = 0;
-        VX_HIP(dev_malloc(&ctx->taa_off, masks * sizeof(uint64_t)));
-        ctx->taa_off_cap = masks;
+        ctx->taa_off_px = 0;
+        VX_HIP(dev_malloc(&ctx->taa_off, most * sizeof(uint64_t)));
+        ctx->taa_off_px = npx;
     }
     A.off = ctx->taa_off;
     if (A.tile_waves == 16) {
