@@ -127,9 +127,9 @@ def region_tuple(r: L.Region):
 
 def _regions(regions):
     """ctypes array of (x, y, z, w, h, d) regions."""
-    if all(len(r) == 6 for r in regions):
-        a = np.array([tuple(r) for r in regions], np.int64).astype(np.int32)
-        return (L.Region * len(regions)).from_buffer(a)
+    a = np.array([tuple(r) for r in regions]) if all(len(r) == 6 for r in regions) else np.empty(0)
+    if a.dtype.kind in "iu":
+        return (L.Region * len(regions)).from_buffer(a.astype(np.int32))
     return (L.Region * len(regions))(*[L.Region(*r) for r in regions])
 
 
