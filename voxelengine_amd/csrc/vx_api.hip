@@ -938,7 +938,8 @@ static vx_status vx_volume_rebuild_impl(vx_volume* v, const vx_instance* inst, u
         size_t maxu = 0;   // a thread's blocks of model voxels (k_footprint)
         for (int q : batches[b]) {
             const FootprintOp& o = ops[q].op;
-            maxu = std::max(maxu, (size_t)((o.sx + 3) / 4) * ((o.sy + 3) / 4) * (o.axis ? (o.sz + 3) / 4 : o.sz));
+            maxu = std::max(maxu, o.axis ? (size_t)((o.sx + 3) / 4) * ((o.sy + 3) / 4) * ((o.sz + 3) / 4)
+                                         : (size_t)((o.sx + 15) / 16) * ((o.sy + 15) / 16) * ((o.sz + 15) / 16) * 256);
         }
         uint32_t gx = (uint32_t)std::min<size_t>((maxu + 255) / 256, 2048);
         for (size_t c0 = 0; c0 < batches[b].size() && e == hipSuccess; c0 += 65535) {

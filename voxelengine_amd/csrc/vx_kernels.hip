@@ -207,7 +207,7 @@ __global__ void k_cells_to_bytes(uint8_t* bytes, const uint64_t* cells, OccView 
 // A thread takes a block of model voxels: 4x4x4 when the operation's transform
 // keeps the axes (op.axis: each coordinate's sum then holds one product and
 // zeros, so the twelve coordinates of the block give all 64 positions), else
-// four rows of four x voxels. Where an axis-keeping block lands on consecutive
+// four rows of four x voxels of a block's 16^3 (footprint_turned). Where an axis-keeping block lands on consecutive
 // voxels inside the volume (always, but for rounding at an integer and the
 // volume's faces) its occupancy is a 64-bit mask that is shifted into the one
 // to eight cell words it covers: one atomic each. Otherwise the per-voxel
@@ -281,12 +281,95 @@ VXD uint32_t footprint_load(const FootprintOp& op, uint32_t xq, uint32_t y, uint
     return m4;
 }
 
+// A turned operation (its transform does not keep the axes) over the 16^3 model
+// voxels at (x0, y0, z0), a block of 256 threads each 4 x 4 x 1 of them. Their
+// voxels' bits meet in a window of cell words in LDS and leave as one atomic per
+// cell: atomics on cells go past the L2, 12 a nanosecond, and bound the launch
+// where a row of four voxels sent its own (67 moved objects, eight launches: 194
+// us so, 108 us with the window). The transform is monotonic in each
+// coordinate, rounding included, so the corners bound the window; one that is too
+// large (a transform that scales) or not finite sends each row's.
+constexpr int32_t kWindowCells = 1024;
+VXD void footprint_turned(uint64_t* cells, const OccView& V, const FootprintOp& op, uint32_t x0, uint32_t y0, uint32_t z0, int32_t thr,
+                          bool dword, bool narrow_cells, uint32_t* window, Footprint& F) {
+    const uint32_t t = threadIdx.x;
+    const uint32_t xq = x0 / 4u + (t & 3u), y = y0 + 4u * ((t >> 2) & 3u), z = z0 + (t >> 4);
+    const uint32_t sx = (uint32_t)op.sx, sy = (uint32_t)op.sy, sz = (uint32_t)op.sz;
+    const float lo[3] = {(float)x0, (float)y0, (float)z0};
+    const float hi[3] = {(float)min(x0 + 15u, sx - 1u), (float)min(y0 + 15u, sy - 1u), (float)min(z0 + 15u, sz - 1u)};
+    const int32_t lim[3] = {2 * V.sx, 2 * V.sy, 2 * V.sz};
+    int32_t c0[3], n[3], total = 1;
+    bool fits = true;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float a = ((op.o[k] + (op.dx[k] < 0.0f ? hi[0] : lo[0]) * op.dx[k]) + (op.dy[k] < 0.0f ? hi[1] : lo[1]) * op.dy[k]) +
+                        (op.dz[k] < 0.0f ? hi[2] : lo[2]) * op.dz[k];
+        const float b = ((op.o[k] + (op.dx[k] < 0.0f ? lo[0] : hi[0]) * op.dx[k]) + (op.dy[k] < 0.0f ? lo[1] : hi[1]) * op.dy[k]) +
+                        (op.dz[k] < 0.0f ? lo[2] : hi[2]) * op.dz[k];
+        fits = fits && fabsf(a) < 1.0e6f && fabsf(b) < 1.0e6f;
+        const int32_t f0 = max(f2i(a * 10.0f), 0), f1 = min(f2i(b * 10.0f), lim[k] - 1);
+        c0[k] = f0 >> 2;
+        n[k] = max((f1 >> 2) - c0[k] + 1, 0);
+        fits = fits && n[k] <= kWindowCells;
+        total = fits ? total * n[k] : 0;
+        fits = fits && total <= kWindowCells;
+    }
+    if (fits)   // (block-uniform)
+        for (int32_t w = (int32_t)t; w < 2 * total; w += 256) window[w] = 0u;
+    __syncthreads();
+    const uint32_t nvalid = 4u * xq < sx ? min(4u, sx - 4u * xq) : 0u;
+    uint32_t m[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) m[i] = nvalid != 0u && y + i < sy && z < sz ? footprint_load(op, xq, y + i, z, nvalid, dword) : 0u;
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+        if (nvalid == 0u || y + i >= sy || z >= sz) break;
+        const uint32_t occ = footprint_occ(i == 0 ? m[0] : (i == 1 ? m[1] : (i == 2 ? m[2] : m[3])), nvalid, thr);
+        if (occ == 0u) continue;
+        if (!fits) {
+            footprint_row(reinterpret_cast<uint32_t*>(cells), V, op, xq, y + i, z, occ, narrow_cells, F);
+            continue;
+        }
+        const float fy = (float)(int32_t)(y + i), fz = (float)(int32_t)z;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (!((occ >> j) & 1u)) continue;
+            const float fx = (float)(int32_t)(4 * xq + j);
+            int32_t f[3];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const float wp = ((op.o[k] + fx * op.dx[k]) + fy * op.dy[k]) + fz * op.dz[k];
+                f[k] = f2i(wp * 10.0f);
+                F.mn[k] = min(F.mn[k], f[k]);
+                F.mx[k] = max(F.mx[k], f[k]);
+            }
+            // SetVolumeAt (ShadowVoxSystem.cpp:82-94): out-of-range writes are dropped.
+            if ((uint32_t)f[0] >= (uint32_t)lim[0] || (uint32_t)f[1] >= (uint32_t)lim[1] || (uint32_t)f[2] >= (uint32_t)lim[2]) continue;
+            const uint32_t bit = cell_bit(f[0], f[1], f[2]);
+            const int32_t w = (((f[2] >> 2) - c0[2]) * n[1] + ((f[1] >> 2) - c0[1])) * n[0] + ((f[0] >> 2) - c0[0]);
+            atomicOr(&window[2 * w + (int32_t)(bit >> 5)], 1u << (bit & 31u));
+        }
+    }
+    __syncthreads();
+    if (fits)
+        for (int32_t w = (int32_t)t; w < total; w += 256) {
+            const unsigned long long b = (unsigned long long)window[2 * w] | (unsigned long long)window[2 * w + 1] << 32;
+            if (b == 0ull) continue;
+            const int32_t r = w / n[0], cx = 4 * (c0[0] + w - r * n[0]), cy = 4 * (c0[1] + r % n[1]), cz = 4 * (c0[2] + r / n[1]);
+            unsigned long long* c = reinterpret_cast<unsigned long long*>(cells) +
+                                    (narrow_cells ? (size_t)cell_index32(V, cx, cy, cz) : cell_index(V, cx, cy, cz));
+            if (op.value) atomicOr(c, b);
+            else atomicAnd(c, ~b);
+        }
+    __syncthreads();
+}
+
 __global__ void __launch_bounds__(256) k_footprint(uint64_t* cells, OccView V, const FootprintOp* ops, int32_t* aabb,
                                                    int32_t thr) {
     const FootprintOp op = ops[blockIdx.y];
     const uint32_t qx = ((uint32_t)op.sx + 3u) >> 2, qy = ((uint32_t)op.sy + 3u) >> 2;
     const uint32_t sy = (uint32_t)op.sy, sz = (uint32_t)op.sz;
-    const uint64_t nu = (uint64_t)qx * qy * (op.axis ? (sz + 3u) >> 2 : sz);
+    const uint64_t nu = op.axis ? (uint64_t)qx * qy * ((sz + 3u) >> 2) : 0u;
     // rows of whole quads and a 4-byte aligned model: one dword per quad
     const bool dword = ((uintptr_t)op.model & 3u) == 0 && (op.sx & 3) == 0;
     const bool narrow_cells = (uint64_t)V.bx * (uint64_t)V.by * (uint64_t)V.bz * 16u < (1ull << 31);
@@ -294,6 +377,14 @@ __global__ void __launch_bounds__(256) k_footprint(uint64_t* cells, OccView V, c
 #pragma unroll
     for (int k = 0; k < 3; ++k) { F.mn[k] = INT32_MAX; F.mx[k] = INT32_MIN; }
     uint32_t* words = reinterpret_cast<uint32_t*>(cells);
+    __shared__ uint32_t window_s[2 * kWindowCells];
+    if (!op.axis) {
+        const uint32_t bx = ((uint32_t)op.sx + 15u) >> 4, by = (sy + 15u) >> 4, n = bx * by * ((sz + 15u) >> 4);
+        for (uint32_t b = blockIdx.x; b < n; b += gridDim.x) {
+            const uint32_t r = b / bx;
+            footprint_turned(cells, V, op, 16u * (b - r * bx), 16u * (r % by), 16u * (r / by), thr, dword, narrow_cells, window_s, F);
+        }
+    }
     const uint64_t stride = (uint64_t)gridDim.x * 256u;
     for (uint64_t u = (uint64_t)blockIdx.x * 256u + threadIdx.x; u < nu; u += stride) {
         uint32_t xq, yq, zu;
@@ -309,18 +400,6 @@ __global__ void __launch_bounds__(256) k_footprint(uint64_t* cells, OccView V, c
             yq = r - zu * qy;
         }
         const uint32_t nvalid = min(4u, (uint32_t)op.sx - 4u * xq);
-        if (!op.axis) {
-            uint32_t m[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) m[i] = 4u * yq + i < sy ? footprint_load(op, xq, 4u * yq + i, zu, nvalid, dword) : 0u;
-#pragma unroll 1
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t mi = i == 0 ? m[0] : (i == 1 ? m[1] : (i == 2 ? m[2] : m[3]));
-                const uint32_t occ = 4u * yq + i < sy ? footprint_occ(mi, nvalid, thr) : 0u;
-                if (occ) footprint_row(words, V, op, xq, 4u * yq + i, zu, occ, narrow_cells, F);
-            }
-            continue;
-        }
         // voxel (j, i, k) of the block is bit j + 4 i + 16 k of M
         uint64_t M = 0;
         uint32_t m[16];
