@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "vx_internal.hpp"
+#include "vx_launch.hpp"
 
 using namespace vx;
 
@@ -709,16 +710,22 @@ extern "C" vx_status vx_volume_clear(vx_volume* v, void* stream) {
     for (int k = 0; k < 2 + v->nlevels; ++k) {
         A.p[k] = p[k];
         A.words[k] = k == 0 ? v->ncells : (k == 1 ? v->ncells / 8 : (size_t)v->wx[k - 2] * v->wy[k - 2] * v->wz[k - 2]);
-        A.blocks[k] = cdiv(A.words[k], 512);
+        A.blocks[k] = (uint32_t)clear_blocks(A.words[k]);
         blocks += A.blocks[k];
     }
     A.grid = v->grid;
     A.ngrid = v->ngrid;
     A.gx = v->gx;
     A.gy = v->gy;
-    blocks += cdiv(v->ngrid, 256);
-    hipLaunchKernelGGL(k_clear_volume, dim3((uint32_t)blocks), dim3(256), 0, S(stream), A, occ_view(v));
-    VX_LAUNCHED("k_clear_volume");
+    blocks += clear_grid_blocks(v->ngrid);
+    hipError_t e = hipSuccess;
+    launch_pieces(blocks, [&](uint32_t first, uint32_t count) {
+        A.first = first;
+        hipLaunchKernelGGL(k_clear_volume, dim3(count), dim3(256), 0, S(stream), A, occ_view(v));
+        e = launch_status();
+        return e == hipSuccess;
+    });
+    if (e != hipSuccess) return fail(VX_ERR_DEVICE, "launch of k_clear_volume failed: %s", hipGetErrorString(e));
     return VX_OK;
 }
 

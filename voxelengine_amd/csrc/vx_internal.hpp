@@ -28,6 +28,7 @@ struct LevelRanges {
 
 // The arrays of a volume (cells, texels, levels 1..3, march grid) to be emptied.
 struct ClearArgs {
+    uint32_t first;                    // the launch's first block
     uint64_t* p[5];
     size_t words[5];
     uint32_t blocks[5];                // 512 words each

@@ -2180,9 +2180,11 @@ __global__ void __launch_bounds__(256) k_mgrid(MgridArgs A, OccView V) {
 
 // An empty volume in one launch: cells, texels and levels zero (16-byte stores),
 // march grid words holding the out-of-bounds bits alone. Blocks of 512 words of
-// the cells, then of the texels, then of each level, then of 256 grid words.
+// the cells, then of the texels, then of each level, then of 256 grid words; a
+// volume of more of them than a launch takes (launch_pieces: from about 2.8e9
+// cell words on) is emptied by two.
 __global__ void __launch_bounds__(256) k_clear_volume(ClearArgs A, OccView V) {
-    uint32_t b = blockIdx.x;
+    uint32_t b = A.first + blockIdx.x;
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
         const uint32_t nb = A.blocks[k];
