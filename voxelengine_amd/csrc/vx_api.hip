@@ -1594,8 +1594,9 @@ static vx_status launch_trace_march_noalloc(vx_ctx* ctx, const vx_volume* vol, c
 }
 
 // A whole view with k_trace_tile, `waves` waves per tile: one kernel, no scratch.
+// `timed`: its time counts for vx_ctx_profile (vx_trace_noalloc's does not).
 static vx_status launch_trace_tile_view(vx_ctx* ctx, const vx_volume* vol, const TraceArgs& T, const TileGeom& g,
-                                        uint32_t waves, hipStream_t stream) {
+                                        uint32_t waves, bool timed, hipStream_t stream) {
     MarchArgs A;
     std::memset(&A, 0, sizeof(A));
     A.item0 = make_march_item(vol, T, 0u, g);
@@ -1611,7 +1612,7 @@ static vx_status launch_trace_tile_view(vx_ctx* ctx, const vx_volume* vol, const
         sparse = sparse || (n[k] > 0 && m[k] != VX_MARCH_DDA);
     }
     hipEvent_t e0 = nullptr, e1 = nullptr;
-    if (ctx->profile && !sparse)
+    if (ctx->profile && timed && !sparse)
         if (vx_status st = profile_events(ctx, e0, e1)) return st;
     hipError_t e = e0 ? hipEventRecord(e0, stream) : hipSuccess;
     if (e == hipSuccess) e = launch_trace_tile(dda, sparse, waves, stream, A);
@@ -1667,7 +1668,7 @@ static vx_status trace_impl(vx_ctx* ctx, const vx_volume* vol, const vx_view* vi
     if (ctx->tuning.kernel == 0 && !A.fetches) {
         const TileGeom g = tile_geom(ctx->tuning, view->width, view->height);
         const uint32_t waves = trace_tile_waves(g.ntiles, params->n_shadow + params->n_ao + params->n_spec, all_dda);
-        if (waves) return launch_trace_tile_view(ctx, vol, A, g, waves, S(stream));
+        if (waves) return launch_trace_tile_view(ctx, vol, A, g, waves, !noalloc, S(stream));
     }
     if (all_dda && ctx->tuning.kernel != 1)
         return noalloc ? launch_trace_march_noalloc(ctx, vol, A, S(stream)) : launch_trace_march(ctx, vol, A, S(stream));
