@@ -187,7 +187,8 @@ struct vx_ctx {
     int32_t device;
     GridCache gcache;
     uint8_t* noalloc;        // this device's vx_trace_noalloc scratch (device address)
-    long long* grad_acc;     // 256*6+6 fixed-point gradient accumulator
+    long long* grad_acc;     // 256*6+6 fixed-point gradient accumulator (adjoint_sum)
+    bool grad_dirty;         // a failed call may have left sums in it
     ShadeArgs* shade_items;  // batched adjoint: per-view arguments (device)
     uint32_t* shade_block0;  // and each view's first block (n + 1 entries)
     uint32_t shade_cap;
@@ -381,6 +382,7 @@ extern "C" vx_status vx_ctx_create(int32_t device, vx_ctx** out) {
     c->gcache.cus = cus;
     c->noalloc = noalloc;
     c->grad_acc = nullptr;
+    c->grad_dirty = false;
     c->shade_items = nullptr;
     c->shade_block0 = nullptr;
     c->shade_cap = 0;
@@ -410,8 +412,9 @@ extern "C" vx_status vx_ctx_create(int32_t device, vx_ctx** out) {
     c->rb_ops = nullptr;
     c->rb_ops_cap = 0;
     hipError_t me = dev_malloc(&c->grad_acc, (256 * 6 + 6) * sizeof(long long));
-    // (the adjoint's accumulator: 0 before a call, cleared by its last kernel)
+    // (0 before the first call on any stream: a non-blocking one does not wait for the null stream)
     if (me == hipSuccess) me = hipMemset(c->grad_acc, 0, (256 * 6 + 6) * sizeof(long long));
+    if (me == hipSuccess) me = hipStreamSynchronize(nullptr);
     if (me == hipSuccess) me = dev_malloc(&c->march.counters, kCounterWords * sizeof(uint32_t));
     if (me != hipSuccess) {
         (void)hipFree(c->grad_acc);
@@ -1905,6 +1908,48 @@ extern "C" vx_status vx_shade_forward(vx_ctx* ctx, const vx_view* view, const vx
     return VX_OK;
 }
 
+// The adjoint's two launches: `accumulate` adds into ctx->grad_acc, which is 0
+// between calls, and k_shade_bwd_finish turns it into the gradients and leaves it
+// at 0 again (1280x720: 18.6 us a call, 20.7 with a clearing launch in every call).
+// A call that fails in between clears it, so that neither the next call nor a
+// recorded one adds to its sums; should that launch fail too, the next call clears
+// it first.
+template <class F>
+static vx_status adjoint_sum(vx_ctx* ctx, const char* name, F accumulate, float* dpalette, float* dlight, hipStream_t s) {
+    constexpr int nacc = 256 * 6 + 6;
+    const auto clear = [&] {
+        hipLaunchKernelGGL(k_zero_u32, dim3(cdiv(2 * nacc, 256)), dim3(256), 0, s, reinterpret_cast<uint32_t*>(ctx->grad_acc),
+                           2 * nacc);
+    };
+    const bool dirty = ctx->grad_dirty;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    hipError_t e = hipSuccess;
+    if (dirty) {
+        e = hipStreamIsCapturing(s, &capture);
+        if (e == hipSuccess) {
+            clear();
+            e = launch_status();
+        }
+    }
+    ctx->grad_dirty = true;
+    if (e == hipSuccess) {
+        accumulate();
+        e = launch_status();
+    }
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_shade_bwd_finish, dim3(cdiv(nacc, 256)), dim3(256), 0, s, ctx->grad_acc, dpalette, dlight);
+        e = launch_status();
+    }
+    if (e != hipSuccess) {
+        clear();
+        (void)hipGetLastError();
+        return fail(VX_ERR_DEVICE, "launch of %s failed: %s", name, hipGetErrorString(e));
+    }
+    // (a clearing launch that was only recorded has not cleared anything yet)
+    ctx->grad_dirty = dirty && capture != hipStreamCaptureStatusNone;
+    return VX_OK;
+}
+
 // Blocks of the adjoint of a view: one per CU at most (k_shade_bwd).
 static uint32_t shade_blocks(uint32_t npx) { return std::min<uint32_t>(cdiv(npx, 1024), 256); }
 
@@ -1916,12 +1961,9 @@ extern "C" vx_status vx_shade_backward(vx_ctx* ctx, const vx_view* view, const v
     if (vx_status st = shade_args(view, g, vis, ssao, palette, light, A)) return st;
     if (vx_status st = use_device(ctx)) return st;
     A.dl_drgb = dl_drgb;
-    const int nacc = 256 * 6 + 6;
-    hipLaunchKernelGGL(k_shade_bwd, dim3(shade_blocks(A.npx)), dim3(1024), 0, S(stream), A, ctx->grad_acc);
-    hipLaunchKernelGGL(k_shade_bwd_finish, dim3(cdiv(nacc, 256)), dim3(256), 0, S(stream), ctx->grad_acc, dpalette,
-                       dlight);
-    VX_LAUNCHED("k_shade_bwd");
-    return VX_OK;
+    return adjoint_sum(ctx, "k_shade_bwd", [&] {
+        hipLaunchKernelGGL(k_shade_bwd, dim3(shade_blocks(A.npx)), dim3(1024), 0, S(stream), A, ctx->grad_acc);
+    }, dpalette, dlight, S(stream));
 }
 
 static vx_status vx_shade_backward_batch_impl(vx_ctx* ctx, const vx_shade_item* items, uint32_t n,
@@ -1957,13 +1999,10 @@ static vx_status vx_shade_backward_batch_impl(vx_ctx* ctx, const vx_shade_item* 
     VX_HIP(hipMemcpyAsync(ctx->shade_items, h.data(), n * sizeof(ShadeArgs), hipMemcpyHostToDevice, S(stream)));
     VX_HIP(hipMemcpyAsync(ctx->shade_block0, b0.data(), (n + 1) * sizeof(uint32_t), hipMemcpyHostToDevice,
                           S(stream)));
-    const int nacc = 256 * 6 + 6;
-    hipLaunchKernelGGL(k_shade_bwd_batch, dim3((uint32_t)blocks), dim3(1024), 0, S(stream), ctx->shade_items,
-                       ctx->shade_block0, n, ctx->grad_acc);
-    hipLaunchKernelGGL(k_shade_bwd_finish, dim3(cdiv(nacc, 256)), dim3(256), 0, S(stream), ctx->grad_acc, dpalette,
-                       dlight);
-    VX_LAUNCHED("k_shade_bwd_batch");
-    return VX_OK;
+    return adjoint_sum(ctx, "k_shade_bwd_batch", [&] {
+        hipLaunchKernelGGL(k_shade_bwd_batch, dim3((uint32_t)blocks), dim3(1024), 0, S(stream), ctx->shade_items,
+                           ctx->shade_block0, n, ctx->grad_acc);
+    }, dpalette, dlight, S(stream));
 }
 
 // ---------------------------------------------------------------------------
