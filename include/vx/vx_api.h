@@ -161,7 +161,9 @@ typedef struct {
  * launch shape is one full-screen draw per pass). 0 / -1 fields mean "default";
  * the autotuner (voxelengine_amd/autotune.py) picks values per workload. */
 typedef struct {
-    int32_t kernel;          /* 0 auto, 1 per-pixel 16x16 tiles, 2 ray-parallel DDA (all-DDA rays only) */
+    int32_t kernel;          /* 0 auto, 1 per-pixel 16x16 tiles, 2 ray-parallel DDA (all-DDA rays only).
+                                Auto: a launch of few rays without fetch counts or hit records takes one
+                                kernel, a block per tile (only auto does); others 2 if all rays are DDA, else 1 */
     int32_t block;           /* ray-parallel kernel threads per block: 256 or 512 (0 = 256) */
     int32_t blocks_per_cu;   /* persistent grid = CUs x this (0 = occupancy limit) */
     int32_t refill;          /* lanes without a running ray that trigger a refill, 1..64 (0 = 16) */
@@ -192,10 +194,11 @@ vx_status vx_ctx_destroy(vx_ctx* ctx);
 vx_status vx_ctx_set_trace_tuning(vx_ctx* ctx, const vx_trace_tuning* tuning);
 vx_status vx_ctx_get_trace_tuning(const vx_ctx* ctx, vx_trace_tuning* tuning);
 /* Kernel timing of the ray-parallel trace (no counterpart in the reference):
- * while enabled, every vx_trace / vx_batch_launch_direct records HIP events
- * around its march kernel on the launch stream. vx_ctx_profile(ctx, 1) starts
- * a new collection, 0 stops it; vx_ctx_profile_read waits for the recorded
- * launches and returns their total march-kernel milliseconds and count. */
+ * while enabled, every vx_trace / vx_batch_launch_direct whose rays are all DDA
+ * records HIP events around its march kernel on the launch stream (a small
+ * vx_trace is one kernel). vx_ctx_profile(ctx, 1) starts a new collection, 0
+ * stops it; vx_ctx_profile_read waits for the recorded launches and returns
+ * their total march-kernel milliseconds and count. */
 vx_status vx_ctx_profile(vx_ctx* ctx, int32_t enable);
 vx_status vx_ctx_profile_read(vx_ctx* ctx, double* march_ms, uint32_t* launches);
 

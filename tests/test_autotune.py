@@ -81,3 +81,40 @@ def test_workload_key_names_the_shape():
     p = configs.trace_params(n_ao=8, n_spec=0)
     k = autotune.workload_key((64, 72, 80), 2, 640, 360, p, device_name="dev")
     assert k == "dev|64x72x80|L2|640x360|1+8+0|m000"
+
+
+def test_the_librarys_own_choice_is_a_candidate(tmp_path):
+    """Only kernel 0 takes the one-kernel trace of small launches: without it as
+    a candidate a tuned small view is slower than an untuned one."""
+    assert dict(kernel=0) in autotune.CANDIDATES
+    assert all(c["kernel"] == 2 for c in autotune.BATCH_CANDIDATES)   # (batches have one kernel)
+    ctx = FakeCtx()
+    best, times = autotune.tune(ctx, lambda: None, "small", cache_path=str(tmp_path / "t.json"),
+                                timer=lambda run, reps: 0.02 if ctx.tuning == dict(kernel=0) else 0.12)
+    assert best == dict(kernel=0) and ctx.tuning == best and len(times) == len(autotune.CANDIDATES)
+
+
+def test_choices_cached_from_the_list_without_it_are_searched_again(tmp_path):
+    path = str(tmp_path / "t.json")
+    before = [dict(kernel=1)] + autotune.MARCH_CANDIDATES
+    other = autotune.MARCH_CANDIDATES[:2]
+    entry = lambda cands: {"tuning": cands[1], "ms": {"0": 2.0, "1": 1.0}, "candidates": cands}
+    json.dump({"a": entry(before), "b": entry(other), "c": {"tuning": dict(kernel=1), "ms": {}}}, open(path, "w"))
+    ctx = FakeCtx()
+    timed = []
+
+    def timer(run, reps):
+        timed.append(1)
+        return 1.0 if ctx.tuning == dict(kernel=0) else 2.0
+
+    best, _ = autotune.tune(ctx, lambda: None, "a", cache_path=path, timer=timer)
+    assert best == dict(kernel=0) and len(timed) == len(autotune.CANDIDATES)
+    assert json.load(open(path))["a"]["candidates"] == autotune.CANDIDATES
+    # searched over a caller's own list, or with no list recorded: as it is cached
+    del timed[:]
+    assert autotune.tune(ctx, lambda: None, "a", cache_path=path, timer=timer)[0] == dict(kernel=0)
+    assert autotune.tune(ctx, lambda: None, "b", cache_path=path, timer=timer)[0] == other[1]
+    assert autotune.tune(ctx, lambda: None, "c", cache_path=path, timer=timer)[0] == dict(kernel=1)
+    json.dump({"a": entry(before)}, open(path, "w"))
+    assert autotune.tune(ctx, lambda: None, "a", candidates=before, cache_path=path, timer=timer)[0] == before[1]
+    assert not timed

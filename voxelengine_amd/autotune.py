@@ -7,10 +7,12 @@ knobs are the tile shape (8x8, 16x4 or 4x16 pixels per 64-ray batch), the
 tile queue order (rows of tiles, or rows of 8x8-tile blocks so that the tiles
 an XCD takes in turn cover a square screen region) and the queue items per
 tile (the library's own choice from the launch's size, one item per tile, or
-three); for a plain trace the per-pixel kernel is a candidate too. Every candidate computes identical bits; only the
-time differs. A batched launch is captured with the tuning current when it
-is created, so tune_batch creates one batch per candidate and returns the
-fastest one.
+three); for a plain trace the per-pixel kernel and the library's own choice are
+candidates too. Only that choice (kernel 0) takes the one-kernel trace of small
+launches (61x43 pixels of 512^3, 18 rays: 46 us, the best of the others 61; with
+the reference's marchers 23 and 74 us). Every candidate computes identical bits; only the time differs. A batched
+launch is captured with the tuning current when it is created, so tune_batch
+creates one batch per candidate and returns the fastest one.
 """
 from __future__ import annotations
 
@@ -23,7 +25,10 @@ DEFAULT_CACHE = os.path.join(os.path.expanduser("~"), ".cache", "voxelengine_amd
 # tile shape x queue order x queue items per tile (0: the library's choice)
 MARCH_CANDIDATES = [dict(kernel=2, tile=t, order=o, chunks=c)
                     for t, o, c in itertools.product((0, 1, 2), (0, 1), (0, 1, 3))]
-CANDIDATES = [dict(kernel=1)] + MARCH_CANDIDATES
+CANDIDATES = [dict(kernel=1)] + MARCH_CANDIDATES + [dict(kernel=0)]
+# the default list before the library's own choice was in it: what a cache holds
+# from a search over it is searched again
+_WITHOUT_AUTO = CANDIDATES[:-1]
 BATCH_CANDIDATES = [c for c in MARCH_CANDIDATES if c["chunks"] == 0]
 
 
@@ -98,7 +103,7 @@ def tune(ctx, run, key: str, candidates=None, cache_path=None, reps=3, force=Fal
     and returns (tuning dict, {candidate index: ms})."""
     cache_path = cache_path or os.environ.get("VX_TUNE_CACHE", DEFAULT_CACHE)
     cache, hit = _cached(cache_path, key, force)
-    if hit:
+    if hit and not (candidates is None and hit.get("candidates") == _WITHOUT_AUTO):
         ctx.set_tuning(**hit["tuning"])
         return hit["tuning"], hit.get("ms", {})
     candidates = candidates or CANDIDATES
