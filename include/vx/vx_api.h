@@ -419,7 +419,7 @@ typedef struct {
  * last position left the screen average a 19x19 same-surface neighbourhood.
  * Uses view width/height and frame; seed keys the per-pixel spiral angle. An out
  * that overlaps an input other than last is written through scratch (16 bytes
- * per pixel, allocated by the first such call). */
+ * per pixel, allocated by the first call for so many pixels, overlapping or not). */
 vx_status vx_light_taa(vx_ctx* ctx, const vx_view* view, const vx_taa_io* io, uint32_t seed, void* stream);
 
 /* ---------------------------------------------------------------- reflection pass

@@ -203,9 +203,8 @@ struct vx_ctx {
     uint32_t* tile_counts;
     uint32_t tile_cap;
     float* taa_out;          // LightTAA: the output of a pass that overwrites one of its inputs
-    uint32_t taa_cap;
     uint64_t* taa_off;       // LightTAA: masks of the pixels whose history lies off the image
-    uint32_t taa_off_px;     // enough of them for images of this many pixels
+    uint32_t taa_px;         // enough of both for images of this many pixels
     // light pass ray list: per pixel first record and count, the total, the records
     uint32_t* lt_first;
     uint32_t* lt_count;
@@ -396,9 +395,8 @@ extern "C" vx_status vx_ctx_create(int32_t device, vx_ctx** out) {
     c->tile_counts = nullptr;
     c->tile_cap = 0;
     c->taa_out = nullptr;
-    c->taa_cap = 0;
     c->taa_off = nullptr;
-    c->taa_off_px = 0;
+    c->taa_px = 0;
     c->lt_first = c->lt_count = c->lt_total = nullptr;
     c->lt_px_cap = 0;
     c->lt_rec = nullptr;
@@ -1340,13 +1338,20 @@ extern "C" vx_status vx_light_taa(vx_ctx* ctx, const vx_view* view, const vx_taa
     const size_t n = npx;
     const bool staged = overlaps(io->light, n * 12) || overlaps(io->motion, n * 8) || overlaps(io->depth, n * 4) ||
                         overlaps(io->normal, n * 12) || overlaps(io->material, n) || overlaps(io->palette, 256 * 24);
-    if (staged && ctx->taa_cap < npx) {
+    // The first call of a size allocates for every later one, overlapping or not, so
+    // that those can be recorded into a graph.
+    if (ctx->taa_px < npx) {
+        // masks of any image of npx pixels: (w / 32 + 1) (h / 32 + 1) 16 at most
+        const size_t most = npx / 64u + (16386u + npx / 16384u) / 2u + 64u;
         VX_HIP(hipDeviceSynchronize());
+        (void)hipFree(ctx->taa_off);
         (void)hipFree(ctx->taa_out);
+        ctx->taa_off = nullptr;
         ctx->taa_out = nullptr;
-        ctx->taa_cap = 0;
+        ctx->taa_px = 0;
+        VX_HIP(dev_malloc(&ctx->taa_off, most * sizeof(uint64_t)));
         VX_HIP(dev_malloc(&ctx->taa_out, n * 16));
-        ctx->taa_cap = npx;
+        ctx->taa_px = npx;
     }
     if (staged) A.out = ctx->taa_out;
     A.tiles = tile_map(view->width, view->height, 16);
@@ -1356,16 +1361,6 @@ extern "C" vx_status vx_light_taa(vx_ctx* ctx, const vx_view* view, const vx_taa
         A.tile_waves = 16;
     }
     const uint32_t masks = A.tiles.ntiles * (uint32_t)A.tile_waves;
-    if (ctx->taa_off_px < npx) {
-        // masks of any image of npx pixels: (w / 32 + 1) (h / 32 + 1) 16 at most
-        const size_t most = npx / 64u + (16386u + npx / 16384u) / 2u + 64u;
-        VX_HIP(hipDeviceSynchronize());
-        (void)hipFree(ctx->taa_off);
-        ctx->taa_off = nullptr;
-        ctx->taa_off_px = 0;
-        VX_HIP(dev_malloc(&ctx->taa_off, most * sizeof(uint64_t)));
-        ctx->taa_off_px = npx;
-    }
     A.off = ctx->taa_off;
     if (A.tile_waves == 16) {
         hipLaunchKernelGGL(k_light_taa32, dim3(A.tiles.blocks), dim3(1024), 0, S(stream), A);
