@@ -6,6 +6,7 @@ missing library or device raises instead of falling back.
 from __future__ import annotations
 
 import ctypes as C
+import struct
 
 import numpy as np
 import torch
@@ -209,6 +210,7 @@ class Volume:
 
 
 _MATRICES = ("last_view", "view", "inv_view", "proj", "inv_proj")
+_F9 = struct.Struct("<9f")
 
 
 def view_struct(vd: dict) -> L.View:
@@ -216,9 +218,13 @@ def view_struct(vd: dict) -> L.View:
     mats = [vd[k] for k in _MATRICES]
     if not all(type(m) is np.ndarray and m.dtype == np.float32 and m.size == 16 for m in mats):
         mats = [np.asarray(m, np.float32).reshape(16) for m in mats]
-    (rx, ry), (ix, iy), (x, y, z), (jx, jy) = vd["res"], vd["ires"], vd["cam_pos"], vd["jitter"]
-    rest = np.array((rx, ry, ix, iy, x, y, z, jx, jy), np.float32)
-    v = L.View.from_buffer_copy(b"".join([m.tobytes() for m in mats]) + rest.tobytes() + bytes(12))
+    vecs = tuple(vd["res"]), tuple(vd["ires"]), tuple(vd["cam_pos"]), tuple(vd["jitter"])
+    try:
+        (rx, ry), (ix, iy), (x, y, z), (jx, jy) = vecs
+        rest = _F9.pack(rx, ry, ix, iy, x, y, z, jx, jy)
+    except Exception:   # fewer elements (the others are 0), text, beyond fp32
+        rest = b"".join([bytes((C.c_float * n)(*[float(e) for e in q])) for n, q in zip((2, 2, 3, 2), vecs)])
+    v = L.View.from_buffer_copy(b"".join([m.tobytes() for m in mats]) + rest + bytes(12))
     v.frame, v.width, v.height = vd["frame"], vd["width"], vd["height"]
     return v
 
