@@ -1,4 +1,5 @@
-"""The forms that view dicts may take: the structures filled as bytes equal those filled element by element through ctypes, and what ctypes
+"""The forms that view dicts and region lists may take: the structures filled as
+bytes equal those filled element by element through ctypes, and what ctypes
 refuses stays refused (host only)."""
 import ctypes as C
 
@@ -53,3 +54,26 @@ def test_refused_views(bad):
         _view_by_elements(vd)
     with pytest.raises(by_elements.type):
         api.view_struct(vd)
+
+
+REGIONS = {
+    "tuples": lambda: [(1, 2, 3, 4, 5, 6), (7, 8, 9, 1, 2, 3)], "iterators": lambda: [iter((1, 2, 3, 4, 5, 6)), map(int, "123456")],
+    "short": lambda: [(1, 2, 3), (1, 2, 3, 4, 5, 6)], "lists": lambda: [[1, 2, 3, 4, 5, 6]], "arrays": lambda: [np.arange(6), np.arange(6, dtype=np.int8)],
+    "truth values": lambda: [(True,) * 6], "negative": lambda: [(-1, -2, -3, 4, 5, 6)], "wide": lambda: [(2 ** 40 + 1, 2, 3, 4, 5, 2 ** 32 - 1)],
+    "wider": lambda: [(2 ** 70 + 1, 2, 3, 4, 5, 6)], "unsigned": lambda: [(np.uint64(2 ** 63 + 3), -2, 3, 4, 5, 6), (np.uint64(3), 2, 3, 4, 5, 6)],
+    "tensors": lambda: [torch.arange(6), tuple(torch.arange(6))],
+    # refused
+    "seven": lambda: [(1, 2, 3, 4, 5, 6, 7)], "floats": lambda: [(1.0, 2, 3, 4, 5, 6)], "texts": lambda: ["123456", ("1", "2", "3", "4", "5", "6")],
+    "nested": lambda: [(np.array([1]),) * 6], "nothing": lambda: [(None,) * 6], "structures": lambda: [L.Region(1, 2, 3, 4, 5, 6)],
+}
+
+
+@pytest.mark.parametrize("name", REGIONS)
+def test_regions(name):
+    try:
+        want = bytes((L.Region * len(REGIONS[name]()))(*[L.Region(*r) for r in REGIONS[name]()]))
+    except Exception as e:
+        with pytest.raises(type(e)):
+            api._regions(REGIONS[name]())
+    else:
+        assert bytes(api._regions(REGIONS[name]())) == want

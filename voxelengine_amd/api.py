@@ -127,10 +127,15 @@ def region_tuple(r: L.Region):
 
 
 def _regions(regions):
-    """ctypes array of (x, y, z, w, h, d) regions."""
-    a = np.array([tuple(r) for r in regions]) if all(len(r) == 6 for r in regions) else np.empty(0)
-    if a.dtype.kind in "iu":
-        return (L.Region * len(regions)).from_buffer(a.astype(np.int32))
+    """ctypes array of (x, y, z, w, h, d) regions: tuples of whole numbers (what
+    rebuild returns) as one array, any other form by its elements."""
+    if all(type(r) is tuple and len(r) == 6 for r in regions):
+        try:
+            a = np.array(regions)
+        except (TypeError, ValueError):   # elements that numpy does not take
+            a = None
+        if a is not None and a.ndim == 2 and a.dtype.kind in "iu":
+            return (L.Region * len(regions)).from_buffer(a.astype(np.int32))
     return (L.Region * len(regions))(*[L.Region(*r) for r in regions])
 
 
