@@ -1307,9 +1307,8 @@ static vx_status vx_primary_instances_impl(vx_ctx* ctx, const vx_vox_cmd* cmds, 
 }
 
 // Tiles of 16 pixels that the 256 CUs hold at once (two a CU): up to there an
-// image takes them, above it tiles of 32. 200x150: 25 us against 32 with tiles
-// of 32, 400x300: 29 / 37, 640x480: 79 / 66, 960x540: 102 / 73, 1920x1080: 333 / 245
-// (measured before both took a tenth less).
+// image takes them, above it tiles of 32. 200x150: 21 us against 28 with tiles
+// of 32, 400x300: 27 / 34, 640x480: 64 / 57, 960x540: 84 / 67, 1920x1080: 285 / 221.
 constexpr uint32_t kTaaSmallTiles = 512;
 
 extern "C" vx_status vx_light_taa(vx_ctx* ctx, const vx_view* view, const vx_taa_io* io, uint32_t seed,

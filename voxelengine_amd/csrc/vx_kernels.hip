@@ -195,9 +195,8 @@ __global__ void k_cells_to_bytes(uint8_t* bytes, const uint64_t* cells, OccView 
     int32_t tx = (int32_t)(i % V.sx);
     int32_t ty = (int32_t)((i / V.sx) % V.sy);
     int32_t tz = (int32_t)(i / ((size_t)V.sx * V.sy));
-    OccView W = V;
-    W.cells = cells;
-    bytes[i] = (uint8_t)texel_byte(W, tx, ty, tz);
+    const size_t ci = brick_index(V, tx >> 2, ty >> 2, tz >> 2) * 8 + sub3(tx >> 1, ty >> 1, tz >> 1);
+    bytes[i] = (uint8_t)gather_byte((uint32_t)(cells[ci] >> texel_base(tx, ty, tz)));
 }
 
 // One footprint loop of ShadowVoxSystem::OnUpdate / OnVoxDestroyed
@@ -1366,8 +1365,9 @@ VXD void add_masked(uint32_t& meta, uint32_t inc, uint64_t m) {
 // wave-uniform: in a batch, a wave that draws a tile of another item first
 // lets its rays in flight finish, then switches.
 // COUNT: every ray's step count is kept for the fetch-count output. Without
-// it the count only serves the 256-step limit, which is tested at block ends,
-// so it advances by STEPS once per block.
+// it the count only serves the 256-step limit: a single view tests it at block
+// ends, so it advances by STEPS once per block; in a batch a pair takes a ray one
+// or two steps, so each is counted.
 template <int BLOCK, int STEPS, bool SINGLE, bool COUNT>
 __global__ void __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(7, 8)))
 k_march(MarchArgs A) {
@@ -2103,19 +2103,17 @@ hipError_t launch_march(int block, int steps, bool single, uint32_t grid, uint32
 }
 
 // Voxels of grid cell (cx, cy, cz) (grid coordinates, border cells included)
-// outside [0, 2s+1], as cell bits; `any_in`: some voxel lies inside.
-VXD uint64_t mgrid_outside(const OccView& V, int32_t cx, int32_t cy, int32_t cz, bool& any_in) {
+// outside [0, 2s+1], as cell bits.
+VXD uint64_t mgrid_outside(const OccView& V, int32_t cx, int32_t cy, int32_t cz) {
     const int32_t f0[3] = {4 * (cx - 1), 4 * (cy - 1), 4 * (cz - 1)};
     const int32_t lim[3] = {2 * V.sx + 1, 2 * V.sy + 1, 2 * V.sz + 1};
     uint32_t om[3];   // bit p: outside along this axis at in-cell position p
-    any_in = true;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
         om[k] = 0;
 #pragma unroll
         for (int p = 0; p < 4; ++p)
             if ((uint32_t)(f0[k] + p) > (uint32_t)lim[k]) om[k] |= 1u << p;
-        any_in = any_in && om[k] != 15u;
     }
     uint64_t w = 0x1111111111111111ull * om[0];
 #pragma unroll
@@ -2158,8 +2156,7 @@ __global__ void __launch_bounds__(256) k_mgrid(MgridArgs A, OccView V) {
         if (inner) {
             A.grid[gi] = __builtin_bitreverse64(cell);
         } else if (cx >= -1 && cy >= -1 && cz >= -1 && cx + 1 < A.gx && cy + 1 < A.gy && cz + 1 < A.gz) {
-            bool any_in;
-            A.grid[gi] = __builtin_bitreverse64(cell | mgrid_outside(V, cx + 1, cy + 1, cz + 1, any_in));
+            A.grid[gi] = __builtin_bitreverse64(cell | mgrid_outside(V, cx + 1, cy + 1, cz + 1));
         }
         // the brick's texels: the cell at x, y, z (0, 1) of it sits 2x + 8y + 32z bits up
         uint32_t h = cell_texels(cell) << (((lane >> 4) & 1u) * 8u + (lane & 1u) * 2u);
@@ -2204,9 +2201,8 @@ __global__ void __launch_bounds__(256) k_clear_volume(ClearArgs A, OccView V) {
     const size_t idx = (size_t)b * 256u + threadIdx.x;
     if (idx >= A.ngrid) return;
     const uint32_t r = (uint32_t)idx / (uint32_t)A.gx, cz = r / (uint32_t)A.gy;
-    bool any_in;
     A.grid[idx] = __builtin_bitreverse64(mgrid_outside(V, (int32_t)((uint32_t)idx - r * (uint32_t)A.gx),
-                                                       (int32_t)(r - cz * (uint32_t)A.gy), (int32_t)cz, any_in));
+                                                       (int32_t)(r - cz * (uint32_t)A.gy), (int32_t)cz));
 }
 
 // ===========================================================================
