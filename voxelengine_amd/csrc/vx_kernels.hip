@@ -669,16 +669,21 @@ VXD void dda_exact(const OccView& V, f3 o, f3 d, float maxt, RayOut& R) {
 // halved. The distances k sf are exact (multiples of 0.5), so positions are
 // counted instead.
 //
-// The march is bound by instructions per position (a Sparse ray takes up to
-// 180): K positions are computed together, which fetches them together, one
-// bounds test serves them (a march is monotonic on every axis), a position's
-// bit is shifted to the sign and one test of the signs' union serves the K. A
+// With a test and a fetch per position the march was bound by instructions (a
+// Sparse ray takes up to 180 positions): K positions are computed together, which
+// fetches them together, one bounds test serves them (a march is monotonic on
+// every axis), a position's bit is shifted to the sign and one test of the signs'
+// union serves the K. A
 // coarse position takes 18 vector instructions on the texel words, a fine one
 // 30 on the march grid, where both took 35 to 40 on the cells with a test each. An axis
 // outside takes texel s, which reads 0 in both. 1 Sparse + 1 SuperSparse ray at
 // 1080p: 260 -> 184 us; 128 lights: 445 -> 323 us. K = 4; with 2 and 8 the lights take 343
 // and 336 us against 330 and reflections 189 and 178 against 170, but the tile
-// trace, whose waves are few, 43 and 31 against 34: it takes 8.
+// trace, whose waves are few, 43 and 31 against 34: it takes 8. What binds now, at
+// 1080p, is the texture path for one ray a pixel (the L1 takes 0.9 accesses a cycle
+// of the one it can; vector issue at 53 % of its ceiling); the lights, whose
+// pixels march several rays one after another, are short of lanes and waves (62 %
+// of a wave's lanes, 3 of 8 waves a SIMD; vector issue 54 %, texture data 68 %).
 constexpr int kSparseAhead = 4;
 
 // First hit among n positions from h on (halved; step d), or -1. h ends n
@@ -2690,7 +2695,9 @@ VXD int32_t intersect_volume_any(const ModelMips& A, const float res[2], int32_t
 // they read, and the step that ends the pass is found by repeating the group.
 // A wave lasts as long as its longest ray (grazing rays step hundreds of
 // voxels at mip 0: up to 150 groups against 25 on average at 1080p), so
-// instructions per step bind: see kPrimarySteps.
+// instructions per step counted most: see kPrimarySteps. As it is, 60 % of the
+// lanes and 4 of 8 waves a SIMD are in use over a 1080p launch, the L1 takes 0.74
+// accesses a cycle and vector issue stands at 40 % of its ceiling.
 VXD bool primary_fast_ok(f3 o, f3 d) {
     const float lo = 7.8886091e-31f;   // 2^-100
     const float dd[3] = {d.x, d.y, d.z}, oo[3] = {o.x, o.y, o.z};
@@ -3454,7 +3461,7 @@ VXD void taa_spiral(const Sampler<T>& S, const Centre& c, size_t i, float u, flo
 // the tile's attributes are gathered from LDS, 40 bytes a texel with the palette
 // beside them (colour and material by index), and a sample's normal, depth and
 // motion are read only where its colour and material are the centre's: 207 us, 16
-// waves a CU (145 KB of LDS a block) with the vector units busy half of it. A sample past
+// waves a CU (145 KB of LDS a block) with vector issue at half its ceiling. A sample past
 // the tile (a variance above 1) reads the G-buffer. Pixels whose history lies
 // off the image are left to k_light_taa_off (A.off: a mask per wave).
 template <int T>
