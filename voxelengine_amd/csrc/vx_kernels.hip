@@ -673,17 +673,17 @@ VXD void dda_exact(const OccView& V, f3 o, f3 d, float maxt, RayOut& R) {
 // Sparse ray takes up to 180 positions): K positions are computed together, which
 // fetches them together, one bounds test serves them (a march is monotonic on
 // every axis), a position's bit is shifted to the sign and one test of the signs'
-// union serves the K. A
-// coarse position takes 18 vector instructions on the texel words, a fine one
-// 30 on the march grid, where both took 35 to 40 on the cells with a test each. An axis
-// outside takes texel s, which reads 0 in both. 1 Sparse + 1 SuperSparse ray at
-// 1080p: 260 -> 184 us; 128 lights: 445 -> 323 us. K = 4; with 2 and 8 the lights take 343
-// and 336 us against 330 and reflections 189 and 178 against 170, but the tile
-// trace, whose waves are few, 43 and 31 against 34: it takes 8. What binds now, at
-// 1080p, is the texture path for one ray a pixel (the L1 takes 0.9 accesses a cycle
-// of the one it can; vector issue at 53 % of its ceiling); the lights, whose
-// pixels march several rays one after another, are short of lanes and waves (62 %
-// of a wave's lanes, 3 of 8 waves a SIMD; vector issue 54 %, texture data 68 %).
+// union serves the K. A coarse position takes 18 vector instructions on the texel
+// words, a fine one 30 on the march grid, where both took 35 to 40 on the cells
+// with a test each. An axis outside takes texel s, which reads 0 in both. 1 Sparse
+// + 1 SuperSparse ray at 1080p: 260 -> 184 us; 128 lights: 445 -> 323 us. K = 4;
+// with 2 and 8 the lights take 343 and 336 us against 330 and reflections 189 and
+// 178 against 170, but the tile trace, whose waves are few, 43 and 31 against 34:
+// it takes 8. What binds now, at 1080p, is the texture path for one ray a pixel
+// (the L1 takes 0.9 accesses a cycle of the one it can; vector issue at 53 % of its
+// ceiling); the lights, whose pixels march several rays one after another, are
+// short of lanes and waves (62 % of a wave's lanes, 3 of 8 waves a SIMD; vector
+// issue 54 %, texture data 68 %).
 constexpr int kSparseAhead = 4;
 
 // First hit among n positions from h on (halved; step d), or -1. h ends n
