@@ -212,7 +212,7 @@ __global__ void k_cells_to_bytes(uint8_t* bytes, const uint64_t* cells, OccView 
 // to eight cell words it covers: one atomic each. Otherwise the per-voxel
 // arithmetic is the reference's, voxel by voxel, and voxels of a row of four
 // that land in the same 32-bit cell word share one atomic.
-// 512^3 identity instance: 72 us (134 MB read), against 330 us voxel by voxel.
+// 512^3 identity instance: 72 to 86 us (134 MB read), against 330 us voxel by voxel.
 struct Footprint {
     int32_t mn[3], mx[3];
 };
@@ -683,7 +683,7 @@ VXD void dda_exact(const OccView& V, f3 o, f3 d, float maxt, RayOut& R) {
 // (the L1 takes 0.9 accesses a cycle of the one it can; vector issue at 53 % of its
 // ceiling); the lights, whose pixels march several rays one after another, are
 // short of lanes and waves (62 % of a wave's lanes, 3 of 8 waves a SIMD; vector
-// issue 54 %, texture data 68 %).
+// issue 54 %, texture data about 70 %).
 constexpr int kSparseAhead = 4;
 
 // First hit among n positions from h on (halved; step d), or -1. h ends n
@@ -2696,8 +2696,8 @@ VXD int32_t intersect_volume_any(const ModelMips& A, const float res[2], int32_t
 // A wave lasts as long as its longest ray (grazing rays step hundreds of
 // voxels at mip 0: up to 150 groups against 25 on average at 1080p), so
 // instructions per step counted most: see kPrimarySteps. As it is, 60 % of the
-// lanes and 4 of 8 waves a SIMD are in use over a 1080p launch, the L1 takes 0.74
-// accesses a cycle and vector issue stands at 40 % of its ceiling.
+// lanes and 4 of 8 waves a SIMD are in use over a 1080p launch, the L1 takes about
+// three accesses in four cycles and vector issue stands at about 40 % of its ceiling.
 VXD bool primary_fast_ok(f3 o, f3 d) {
     const float lo = 7.8886091e-31f;   // 2^-100
     const float dd[3] = {d.x, d.y, d.z}, oo[3] = {o.x, o.y, o.z};
